@@ -1,0 +1,75 @@
+"""Orbits that become cycles of states stop early in the kernels' unchecked blocks;
+counts, smooth values and iteration totals stay those of the full loop, so each
+engine is compared with the oracle (which runs every step) on views with much
+interior, at iteration limits around the first held state, the block ends and the
+first tests.  Counts and iterations are whole numbers and must be equal; smooth
+values are within 1e-12 relative, as in the other kernel tests.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SMOOTH_RTOL = 1e-12
+# around kCycleFirst = 64, block ends, the first held states' tests, and far past them
+LIMITS = [1, 63, 64, 65, 79, 80, 81, 97, 112, 113, 300, 3001]
+VIEWS = {
+    "home": dict(box=(-2.0, -1.25, 0.75, 1.25)),
+    "period3": dict(box=(-1.80, -0.05, -1.72, 0.05)),
+    "axis": dict(box=(-1.5, -0.01, 0.5, 0.01)),  # the real axis: y stays 0 at the middle row
+    "julia_bounded": dict(box=(-1.5, -1.5, 1.5, 1.5), kind=1, julia_c=(-0.12, 0.74)),
+    "julia_zero": dict(box=(-1.25, -1.25, 1.25, 1.25), kind=1, julia_c=(0.0, 0.0)),
+}
+
+
+def tile_of(cu, view, limit, spp, bailout=4.0, size=(53, 37)):
+    v = VIEWS[view]
+    return cu.make_tile(*v["box"], *size, limit, bailout, kind=v.get("kind", 0),
+                        julia_c=v.get("julia_c", (0.0, 0.0)), spp=spp,
+                        pattern=cu.SAMPLE_JITTER if spp > 1 else cu.SAMPLE_CENTRE, seed=limit)
+
+
+def same(got, want):
+    (c, s, it), (wc, ws, wit) = got, want
+    assert np.array_equal(c.reshape(wc.shape), wc)
+    assert it == wit
+    rel = np.abs(s.reshape(ws.shape) - ws) / np.maximum(np.abs(ws), 1.0)
+    assert rel.max() <= SMOOTH_RTOL
+
+
+def grid(cu, engine, tile, precision):
+    n = tile.width * tile.height
+    counts, smooth, iters = cu.DeviceBuffer(n * 4), cu.DeviceBuffer(n * 8), cu.IterationCounter()
+    engine.escape_tile(precision, tile, counts, smooth, iters)
+    cu.synchronize()
+    return counts.download(np.uint32), smooth.download(np.float64), iters.total()
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("spp", [1, 3])
+@pytest.mark.parametrize("view", sorted(VIEWS))
+def test_grid_kernel(gpu, engine, oracle, view, spp, precision):
+    for limit in LIMITS:
+        tile = tile_of(gpu, view, limit, spp)
+        same(grid(gpu, engine, tile, precision), oracle.escape_tile(tile, precision))
+
+
+def deep_case(cu, engine, oracle, desc, method):
+    """A deep frame and the oracle's checked loop over its pixels, bit for bit."""
+    f = cu.DeepFrame(engine, desc, method)
+    f.render()
+    rep, counts = f.report(), f.counts()
+    orbit = f.orbit() if method != cu.DEEP_DIRECT_F64 else None
+    f.close()
+    ys, xs = np.mgrid[0:desc.height, 0:desc.width]
+    om = {cu.DEEP_DIRECT_F64: oracle.DEEP_DIRECT_F64, cu.DEEP_PERTURB_F32: oracle.DEEP_PERTURB_F32,
+          cu.DEEP_PERTURB_F64: oracle.DEEP_PERTURB_F64}[method]
+    wc, _, _, wit = oracle.deep_pixels(om, xs.ravel(), ys.ravel(), desc, orbit, rep.reference_length)
+    assert np.array_equal(counts.ravel(), wc)
+    assert rep.iterations == wit
+
+
+@pytest.mark.parametrize("limit", LIMITS)
+def test_direct_deep_frame(gpu, engine, oracle, limit):
+    deep_case(gpu, engine, oracle, gpu.make_deep(-0.25, 0.125, 1.5, 61, 39, limit, 16.0),
+              gpu.DEEP_DIRECT_F64)

@@ -390,6 +390,10 @@ __device__ __forceinline__ void tile_point<float>(const cu_tile_desc &t, uint px
 // Wave-level helpers (wave64).
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 __device__ __forceinline__ uint lane_id() { return __lane_id(); }
+// Lanes in a wave-uniform mask (a scalar; compared as one).
+__device__ __forceinline__ uint lanes(uint64_t mask) {
+    return (uint)__builtin_amdgcn_readfirstlane(__popcll(mask));
+}
 // The iteration counter is CU_ITER_SLOTS u64 slots; each wave adds its total
 // to one slot chosen by its global wave number, so a launch of a million waves
 // does not serialise on one address.  The caller sums the slots.  All 64 lanes

@@ -73,3 +73,41 @@ def deep_case(cu, engine, oracle, desc, method):
 def test_direct_deep_frame(gpu, engine, oracle, limit):
     deep_case(gpu, engine, oracle, gpu.make_deep(-0.25, 0.125, 1.5, 61, 39, limit, 16.0),
               gpu.DEEP_DIRECT_F64)
+
+
+# (centre, height of the view, precision): the whole set in FP32; FP64 views below the
+# float ulp inside the period-2 disk's edge and inside the period-3 island
+RENDER_VIEWS = [("mandelbrot", (-0.5, 0.0), 2.5, 32), ("mandelbrot", (-1.25, 0.0), 2e-6, 64),
+                ("mandelbrot", (-1.7548777, 0.0), 2e-6, 64), ("julia", (0.0, 0.0), 3.0, 32)]
+
+
+@pytest.mark.parametrize("fractal,centre,zoom,precision", RENDER_VIEWS)
+@pytest.mark.parametrize("samples,adaptive", [(1.0, 0), (4.0, 0), (5.0, 1)])
+def test_module_kernels(gpu, oracle, fractal, centre, zoom, precision, samples, adaptive):
+    """The main kernel's pooled orbits (first held state at 128), FP32 and FP64."""
+    cu, w, h = gpu, 67, 45
+    provider = cu.FractalRendererProvider()
+    r = provider.get_renderer(fractal)
+    kind, jc = (cu.FRACTAL_JULIA, (-0.12, 0.74)) if fractal == "julia" else (cu.FRACTAL_MANDELBROT, (0, 0))
+    if fractal == "julia":
+        r.set_fractal_custom_params("-0.12;0.74")
+    r.initialize_rendering(w, h, cu.default_palette())
+    try:
+        seg = cu.plane_segment_from_center(*centre, zoom, w, h)
+        for limit in LIMITS + [127, 128, 129, 144, 145, 192, 208]:
+            m = cu.RenderingModel()
+            m.set_segment(*seg)
+            m.max_iterations, m.max_super_sampling = limit, samples
+            m.use_adaptive_super_sampling = adaptive
+            before = r.iterations()
+            r.render_quality(m)
+            oracle.render_iterations()
+            want = oracle.render_main(precision, kind, jc, w, h, seg, limit, samples,
+                                      cu.FLAG_ADAPTIVE_SS if adaptive else 0)
+            assert r.iterations() - before == oracle.render_iterations()
+            got = r.read_pixel_info()
+            for field in ("value", "weight", "is_reused", "weight_of_new_samples"):
+                assert np.array_equal(got[field], want[field]), (limit, field)
+    finally:
+        r.free_rendering_resources()
+        provider.close()

@@ -162,6 +162,11 @@ struct Orbit {
 // 1.5 from 128, 0.44 and 0.52 with tests at every second and fourth block end.
 constexpr uint kCycleFirst = 64;
 
+// The same for kernels whose lanes take orbits at different times and hold per lane:
+// from 128 iterations on, an orbit that escapes at the usual depths (136 steps on
+// average in the 4096^2 frame at width 1e-4) seldom pays for a hold.
+constexpr uint kCycleFirstMixed = 128;
+
 // In a wave-uniform branch: keeps it a branch, where the compiler would otherwise
 // run its few instructions as selects on every pass.
 __device__ __forceinline__ void seldom() { asm volatile(""); }
@@ -422,6 +427,96 @@ __device__ __forceinline__ uint skewed_block_x() {
 // becomes the execution mask itself, with no per-lane shift and compare.
 __device__ __forceinline__ bool in_mask(uint64_t mask) {
     return __builtin_amdgcn_inverse_ballot_w64(mask);
+}
+
+// The orbit a lane iterates in the kernels whose lanes take and finish orbits at
+// different times.
+template <class Real>
+struct LaneOrbit {
+    Real x, y, cx, cy;    // state and constant
+    Real sx, sy, mx, my;  // start and midpoint of its last block
+    Real hx, hy;          // held state of the cycle test
+    uint i;               // iterations run (those of a failed block included)
+    uint until;           // count at which the next state is held or the blocks end
+
+    // Starts the block loop at (x, y, i); `first` is the earliest count to hold a state at.
+    template <int K>
+    __device__ __forceinline__ void begin(uint max_iter, uint first) {
+        hx = x;
+        hy = y;
+        until = min(i < first ? first : next_hold<K>(i), max_iter - (uint)K + 1u);
+    }
+};
+
+// Unchecked blocks of K steps for the lanes in `run`, until none runs or at least
+// `enough` of the `counted` lanes do not.  Which lanes run is wave-uniform: a lane
+// leaves `run` for `failed` when its block ends outside (the escape lies in that
+// block), or for `ended` when fewer than K of its max_iter steps are left or, with i
+// set to max_iter, when its orbit has become a cycle of states (escape_orbit has the
+// reason).  A block in which no lane changes costs one branch beyond its steps and
+// three compares: while many waves run the loop is bound by VALU issue, but the few
+// waves left with the longest orbits set a launch's length, and a lone wave waits
+// for every scalar instruction.  Whole wave.
+template <class Real, int K, bool kFused>
+__device__ __forceinline__ void run_blocks(LaneOrbit<Real> &o, uint64_t &run, uint64_t &failed,
+                                           uint64_t &ended, uint64_t counted, uint enough,
+                                           uint max_iter, Real bsq) {
+    Real x2 = o.x * o.x, y2 = o.y * o.y;  // squares of the current state, carried
+    while (run != 0 && lanes(counted & ~run) < enough) {
+        uint64_t inside, due, again;
+        do {
+            if (in_mask(run)) {
+                o.sx = o.x;
+                o.sy = o.y;
+#pragma unroll
+                for (int k = 0; k < K / 2; ++k)
+                    quad_step_sq<Real, kFused>(o.x, o.y, x2, y2, o.cx, o.cy);
+                o.mx = o.x;
+                o.my = o.y;
+#pragma unroll
+                for (int k = K / 2; k < K; ++k)
+                    quad_step_sq<Real, kFused>(o.x, o.y, x2, y2, o.cx, o.cy);
+                o.i += K;
+            }
+            inside = ballot(x2 + y2 < bsq);
+            due = ballot(o.i >= o.until);
+            again = ballot(o.y == o.hy);
+        } while ((run & (~inside | due | again)) == 0);
+        failed |= run & ~inside;
+        run &= inside;
+        if ((run & (due | again)) != 0) {
+            seldom();
+            const uint64_t cycle = run & again & ballot(o.x == o.hx);
+            if (in_mask(cycle)) o.i = max_iter;  // the loop's result: max_iter steps, no escape
+            const uint64_t spent = run & ballot(o.i > max_iter - (uint)K);
+            ended |= spent;
+            run &= ~spent;
+            if (in_mask(run & due)) {
+                o.hx = o.x;
+                o.hy = o.y;
+                o.until = min(next_hold<K>(o.i), max_iter - (uint)K + 1u);
+            }
+        }
+    }
+}
+
+// Exact stop of a lane that run_blocks left in `failed` (its escape lies in its
+// last block) or `ended` (checked steps, if any are left).  o.i becomes the
+// iterations executed; true with the failing |z|^2 when the orbit escaped.
+template <class Real, int K, bool kFused>
+__device__ __forceinline__ bool finish_orbit(LaneOrbit<Real> &o, uint64_t failed, uint max_iter,
+                                             Real bsq, Real &mag2) {
+    bool escaped = false;
+    mag2 = 0;
+    if (in_mask(failed)) {
+        // a failing test at max_iter itself is never reached by the reference loop
+        o.i = locate_escape<Real, K, kFused>(o.x, o.y, o.sx, o.sy, o.mx, o.my, o.cx, o.cy,
+                                             o.i - (uint)K, bsq, mag2);
+        escaped = o.i < max_iter;
+    } else {
+        checked_steps<Real, kFused>(o.x, o.y, o.cx, o.cy, o.i, max_iter, bsq, escaped, mag2);
+    }
+    return escaped;
 }
 
 }  // namespace cu

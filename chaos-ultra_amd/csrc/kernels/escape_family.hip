@@ -148,16 +148,21 @@ __device__ void escape_tile_samples(const cu_tile_desc &t, double smooth_c, uint
 // ---------------------------------------------------------------------------
 // persistent lane-refill launch over many tiles
 // ---------------------------------------------------------------------------
-// Every wave keeps 64 independent samples in flight.  Lanes run unchecked
-// blocks of K steps in lock step; a lane whose block fails its end test (or
-// whose remaining budget is below K) becomes pending.  Once `refill` lanes are
-// pending or idle, the pending lanes locate the exact escape step in the half of
-// their last block that holds it (cu::locate_escape), finish their sample, start the next sample of the same
+// Every wave keeps 64 independent samples in flight.  Lanes run unchecked blocks
+// of K steps in lock step (cu::run_blocks); a lane whose block fails its end test,
+// whose remaining budget is below K or whose orbit has become a cycle of states
+// becomes pending.  Once `refill` lanes are pending or idle, the pending lanes locate
+// the exact escape step in the half of their last block that holds it
+// (cu::locate_escape), finish their sample, start the next sample of the same
 // pixel or write the pixel, and idle lanes take new pixels from a wave-private
 // chunk of the global pixel queue (one atomic per `chunk` pixels).  Pixels of
 // one tile are numbered row-major from the tile's work_offset.  There is no
 // barrier after the tile table is staged, and every wave leaves once the queue
 // is exhausted and its lanes are idle.
+//
+// Bound by VALU issue, then by the longest orbits at the end.  Batches of 32 and 24
+// uneven tiles, FP64, tune 32/32/256/16: 7.7 -> 3.0 and 10.0 -> 2.8 ms with the cycle
+// test (1.8e10 and 2.3e10 loop iterations); 32 tiles in FP32 9.4 -> 1.9 ms.
 template <class Real, int K, bool kFused>
 __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, uint n_tiles,
                                         uint64_t total, uint *counts, double *smooth,
@@ -174,11 +179,12 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
     const uint lane = cu::lane_id();
     const uint64_t lanes_below = (1ull << lane) - 1ull;
 
-    int mode = 0;          // 0 idle, 1 running unchecked blocks, 2 pending checked work
-    bool replay = false;   // pending lane's last block failed: locate the escape in it
-    uint tile = 0, px = 0, py = 0, s = 0, i = 0, count_sum = 0;
+    uint64_t run = 0, failed = 0, ended = 0;  // lanes by state (cu::run_blocks); the rest are idle
+    uint64_t able = 0;                        // lanes whose tile can use unchecked blocks
+    cu::LaneOrbit<Real> o = {};
+    Real bsq = 4;
+    uint tile = 0, px = 0, py = 0, s = 0, count_sum = 0;
     double smooth_sum = 0;
-    Real x = 0, y = 0, cx = 0, cy = 0, sx = 0, sy = 0, mx = 0, my = 0, bsq = 4;
     uint max_iter = 0;
     uint64_t executed = 0;
 
@@ -194,7 +200,7 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
 
     for (;;) {
         // ---- refill idle lanes ----
-        uint64_t idle = cu::ballot(mode == 0);
+        uint64_t idle = ~(run | ended);
         while (idle != 0 && !exhausted) {
             if (cur >= end) {
                 unsigned long long base = 0;
@@ -211,7 +217,9 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
             const uint64_t avail = end - cur;
             const uint take = (uint)min((uint64_t)n, avail);
             const uint rank = (uint)__popcll(idle & lanes_below);
-            if (mode == 0 && rank < take) {
+            const uint64_t taken = idle & cu::ballot(rank < take);
+            bool blocks = false;
+            if (cu::in_mask(taken)) {
                 const uint64_t item = cur + rank;
                 uint lo = 0, hi = n_tiles - 1;  // last tile with work_offset <= item
                 while (lo < hi) {
@@ -228,69 +236,48 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
                 smooth_sum = 0;
                 max_iter = t.max_iter;
                 bsq = (Real)t.bailout_sq;
-                begin_sample<Real>(t, px, py, 0, x, y, cx, cy);
-                i = 0;
-                replay = false;
-                mode = (tile_blocks_valid(t) && max_iter >= (uint)K) ? 1 : 2;
+                begin_sample<Real>(t, px, py, 0, o.x, o.y, o.cx, o.cy);
+                o.i = 0;
+                o.template begin<K>(max_iter, cu::kCycleFirstMixed);
+                blocks = tile_blocks_valid(t) && max_iter >= (uint)K;
             }
+            const uint64_t ok = cu::ballot(blocks);
+            able = (able & ~taken) | ok;
+            run |= ok;
+            ended |= taken & ~ok;
             cur += take;
-            idle = cu::ballot(mode == 0);
+            idle &= ~taken;
         }
-        if (cu::ballot(mode != 0) == 0) break;
+        if ((run | ended) == 0) break;
 
-        // ---- unchecked blocks until enough lanes wait ----
-        for (;;) {
-            if (mode == 1) {
-                sx = x;
-                sy = y;
-#pragma unroll
-                for (int k = 0; k < K / 2; ++k) cu::quad_step<Real, kFused>(x, y, cx, cy);
-                mx = x;
-                my = y;
-#pragma unroll
-                for (int k = K / 2; k < K; ++k) cu::quad_step<Real, kFused>(x, y, cx, cy);
-                if (x * x + y * y < bsq) {
-                    i += K;
-                    if (max_iter - i < (uint)K) mode = 2;
-                } else {
-                    mode = 2;
-                    replay = true;
-                }
-            }
-            const uint64_t run = cu::ballot(mode == 1);
-            const uint waiting = (uint)__popcll(cu::ballot(mode == 2)) +
-                                 (exhausted ? 0u : (uint)__popcll(cu::ballot(mode == 0)));
-            if (run == 0 || waiting >= refill) break;
-        }
+        cu::run_blocks<Real, K, kFused>(o, run, failed, ended, exhausted ? run | ended : ~0ull,
+                                        refill, max_iter, bsq);
 
         // ---- pending lanes: locate the escape or run checked steps, finish the sample ----
-        if (mode == 2) {
-            bool escaped = false;
-            Real mag2 = 0;
-            if (replay) {
-                // a failing test at max_iter itself is never reached by the reference loop
-                i = cu::locate_escape<Real, K, kFused>(x, y, sx, sy, mx, my, cx, cy, i, bsq, mag2);
-                escaped = i < max_iter;
-                replay = false;
-            } else {
-                cu::checked_steps<Real, kFused>(x, y, cx, cy, i, max_iter, bsq, escaped, mag2);
-            }
+        bool another = false;
+        if (cu::in_mask(failed | ended)) {
+            Real mag2;
+            const bool escaped = cu::finish_orbit<Real, K, kFused>(o, failed, max_iter, bsq, mag2);
             const cu_tile_desc &t = tiles[tile];
-            executed += i;
-            count_sum += escaped ? i : (t.kind == CU_FRACTAL_JULIA ? max_iter : 0u);
-            smooth_sum += escaped ? cu::smooth_value(i, (double)mag2, lds_smooth_c[tile]) : 0.0;
+            executed += o.i;
+            count_sum += escaped ? o.i : (t.kind == CU_FRACTAL_JULIA ? max_iter : 0u);
+            smooth_sum += escaped ? cu::smooth_value(o.i, (double)mag2, lds_smooth_c[tile]) : 0.0;
             ++s;
             if (s < t.spp) {
-                begin_sample<Real>(t, px, py, s, x, y, cx, cy);
-                i = 0;
-                mode = (tile_blocks_valid(t) && max_iter >= (uint)K) ? 1 : 2;
+                begin_sample<Real>(t, px, py, s, o.x, o.y, o.cx, o.cy);
+                o.i = 0;
+                o.template begin<K>(max_iter, cu::kCycleFirstMixed);
+                another = true;
             } else {
-                const uint64_t o = t.out_offset + (uint64_t)py * t.out_pitch + px;
-                counts[o] = count_sum / t.spp;
-                if (smooth) smooth[o] = smooth_sum / (double)t.spp;
-                mode = 0;
+                const uint64_t at = t.out_offset + (uint64_t)py * t.out_pitch + px;
+                counts[at] = count_sum / t.spp;
+                if (smooth) smooth[at] = smooth_sum / (double)t.spp;
             }
         }
+        const uint64_t more = cu::ballot(another);
+        run |= more & able;
+        ended = more & ~able;
+        failed = 0;
     }
     cu::add_iterations(iters, executed);
 }

@@ -182,10 +182,6 @@ __device__ __forceinline__ uint next_vote_round(uint c, uint n, bool adaptive) {
 // which a wave stops its unchecked blocks to hand out new samples.
 constexpr uint kRing = 4;
 constexpr uint kRefill = 16;
-// First held state of the cycle test here: from 128 iterations on instead of 64, an
-// orbit that escapes at the usual depths (136 steps on average at the 4096^2
-// frame's view) seldom pays for one (4K there, FP64, 4 spp: 1 % less than with 64).
-constexpr uint kPoolCycleFirst = 128;
 constexpr unsigned long long kAbsent = ~0ull;  // above any iteration count
 
 // One wave's LDS: each pixel's results of the rounds not yet voted on
@@ -241,7 +237,6 @@ __device__ uint sample_the_fractal(WaveLds &lds, int site, Point<uint> grid, Rec
     const uint64_t group = half & (site == 1 ? site1 : (site == 2 ? site2 : 0ull));
     const bool blocks = Fractal::blocks_valid(4.0) && max_iter >= (uint)K;
     const Real bsq = (Real)4;
-    const uint last = max_iter - (uint)K;  // a block may start at i <= last
 
     // ---- the pixel this lane owns ----
     bool in_loop = site != 0;
@@ -266,10 +261,8 @@ __device__ uint sample_the_fractal(WaveLds &lds, int site, Point<uint> grid, Rec
     uint64_t run = 0;     // lanes running unchecked blocks
     uint64_t failed = 0;  // lanes whose last block failed its end test (locate the escape)
     uint64_t ended = 0;   // lanes left with checked steps, or at the end of a cycle
-    uint task = lane, i = 0;  // owner lane | sample << 8
-    Real x = 0, y = 0, cx = 0, cy = 0, sx = 0, sy = 0, mx = 0, my = 0;
-    Real hx = 0, hy = 0;  // held state of the cycle test (escape_core.hpp)
-    uint until = 0;       // iteration count at which the next one is held or the blocks end
+    uint task = lane;     // owner lane | sample << 8
+    cu::LaneOrbit<Real> o = {};
     wave_lds_fence();
 
     for (;;) {
@@ -367,71 +360,23 @@ __device__ uint sample_the_fractal(WaveLds &lds, int site, Point<uint> grid, Rec
                     // c = leftTop + (1,-1) * (pixel + delta) * pixelSize  (:119-124)
                     const Real X = image.left_bottom.x + ((Real)op.x + dx) * psx;
                     const Real Y = image.right_top.y - ((Real)op.y + dy) * psy;
-                    Fractal::start<Real>(X, Y, x, y, cx, cy);
-                    i = 0;
-                    hx = x;
-                    hy = y;
-                    until = min(kPoolCycleFirst, last + 1u);
+                    Fractal::start<Real>(X, Y, o.x, o.y, o.cx, o.cy);
+                    o.i = 0;
+                    o.template begin<K>(max_iter, cu::kCycleFirstMixed);
                 }
                 (blocks ? run : ended) |= taken;
             }
         }
 
         // ---- unchecked blocks until kRefill lanes wait (idle ones count while work is left) ----
-        Real x2 = x * x, y2 = y * y;  // squares of the current state, carried
-        const uint64_t counted = more ? ~0ull : run | ended;
-        while (run != 0 && cu::lanes(counted & ~run) < kRefill) {
-            // blocks until some lane's state changes: one branch per block, as the few
-            // waves left with the longest orbits set the launch's length
-            uint64_t inside, due, again;
-            do {
-                if (cu::in_mask(run)) {
-                    sx = x;
-                    sy = y;
-#pragma unroll
-                    for (int k = 0; k < K / 2; ++k)
-                        cu::quad_step_sq<Real, kFused>(x, y, x2, y2, cx, cy);
-                    mx = x;
-                    my = y;
-#pragma unroll
-                    for (int k = K / 2; k < K; ++k)
-                        cu::quad_step_sq<Real, kFused>(x, y, x2, y2, cx, cy);
-                    i += K;
-                }
-                inside = cu::ballot(x2 + y2 < bsq);
-                due = cu::ballot(i >= until);
-                again = cu::ballot(y == hy);
-            } while ((run & (~inside | due | again)) == 0);
-            failed |= run & ~inside;
-            run &= inside;
-            if ((run & (due | again)) != 0) {
-                cu::seldom();
-                const uint64_t cycle = run & again & cu::ballot(x == hx);
-                if (cu::in_mask(cycle)) i = max_iter;  // maxIter steps, no escape
-                const uint64_t spent = run & cu::ballot(i > last);
-                ended |= spent;
-                run &= ~spent;
-                if (cu::in_mask(run & due)) {
-                    hx = x;
-                    hy = y;
-                    until = min(cu::next_hold<K>(i), last + 1u);
-                }
-            }
-        }
+        cu::run_blocks<Real, K, kFused>(o, run, failed, ended, more ? ~0ull : run | ended, kRefill,
+                                        max_iter, bsq);
 
         // ---- finish the pending orbits and post their iteration counts ----
         if (cu::in_mask(failed | ended)) {
-            Real mag2 = 0;
-            if (cu::in_mask(failed)) {
-                // a failing test at max_iter itself is never reached by the reference loop:
-                // n == max_iter then reads as an orbit that did not escape
-                i = cu::locate_escape<Real, K, kFused>(x, y, sx, sy, mx, my, cx, cy, i - (uint)K,
-                                                       bsq, mag2);
-            } else {
-                bool escaped = false;
-                cu::checked_steps<Real, kFused>(x, y, cx, cy, i, max_iter, bsq, escaped, mag2);
-            }
-            lds.result[(task >> 8) % kRing][task & 63u] = (unsigned long long)i;
+            Real mag2;
+            cu::finish_orbit<Real, K, kFused>(o, failed, max_iter, bsq, mag2);
+            lds.result[(task >> 8) % kRing][task & 63u] = (unsigned long long)o.i;
         }
         failed = ended = 0;
         wave_lds_fence();

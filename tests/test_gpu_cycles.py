@@ -111,3 +111,27 @@ def test_module_kernels(gpu, oracle, fractal, centre, zoom, precision, samples, 
     finally:
         r.free_rendering_resources()
         provider.close()
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("spp", [1, 3])
+@pytest.mark.parametrize("steps,chunk,refill", [(8, 64, 1), (16, 256, 16), (32, 100, 64)])
+def test_persistent_kernel(gpu, engine, oracle, steps, chunk, refill, spp, precision):
+    """All views and limits (and one bailout below 4, which takes checked steps) as one batch."""
+    import importlib
+    at = importlib.import_module("chaos-ultra_amd.autotune")
+    limits = LIMITS + [7, 8, 15, 16, 31, 32, 33, 128, 159, 160, 161]
+    tiles = [tile_of(gpu, v, n, spp, size=(29, 17)) for v in sorted(VIEWS) for n in limits]
+    tiles.append(tile_of(gpu, "home", 300, spp, bailout=3.0))
+    batch = at.PersistentBatch(gpu, tiles, precision)
+    batch.render(engine, gpu.Tune(steps, 8, chunk, refill))
+    gpu.synchronize()
+    counts, smooth = batch.counts.download(np.uint32), batch.smooth.download(np.float64)
+    total, offset = 0, 0
+    for t in tiles:
+        n = t.width * t.height
+        wc, ws, wit = oracle.escape_tile(t, precision)
+        same((counts[offset:offset + n], smooth[offset:offset + n], wit), (wc, ws, wit))
+        total += wit
+        offset += n
+    assert batch.iters.total() == total

@@ -67,94 +67,63 @@ constexpr uint kSubQueues = 1024;
 // the drain's time; at 4 the last grabs still share out evenly.
 constexpr uint kDrainGrab = 4;
 
-// Result of a pending lane (its block failed, or it is within K steps of
-// max_iter, or it cannot use blocks): the exact stop, the count in the
-// fractal's computeFractal convention and the smooth value.  i becomes the
-// iterations executed by the sample.
+// Result of a lane that run_blocks left in `failed` or `ended`: the exact stop, the
+// count in the fractal's computeFractal convention and the smooth value.  o.i becomes
+// the iterations executed by the sample.
 template <class Real, int K, bool kFused>
-__device__ __forceinline__ void finish_pending(Real x, Real y, Real sx, Real sy, Real mx, Real my,
-                                               Real cx, Real cy, uint &i, uint max_iter, Real bsq,
-                                               double smooth_c, bool julia, bool replay,
-                                               uint &count, double &smooth) {
-    bool escaped = false;
-    Real mag2 = 0;
-    if (replay) {
-        // a failing test at max_iter itself is never reached by the reference loop
-        i = cu::locate_escape<Real, K, kFused>(x, y, sx, sy, mx, my, cx, cy, i, bsq, mag2);
-        escaped = i < max_iter;
-    } else {
-        cu::checked_steps<Real, kFused>(x, y, cx, cy, i, max_iter, bsq, escaped, mag2);
-    }
-    count = escaped ? i : (julia ? max_iter : 0u);
-    smooth = escaped ? cu::smooth_value(i, (double)mag2, smooth_c) : 0.0;
+__device__ __forceinline__ void finish_sample(cu::LaneOrbit<Real> &o, uint64_t failed,
+                                              uint max_iter, Real bsq, double smooth_c,
+                                              bool julia, uint &count, double &smooth) {
+    Real mag2;
+    const bool escaped = cu::finish_orbit<Real, K, kFused>(o, failed, max_iter, bsq, mag2);
+    count = escaped ? o.i : (julia ? max_iter : 0u);
+    smooth = escaped ? cu::smooth_value(o.i, (double)mag2, smooth_c) : 0.0;
 }
 
 // Orbit of one lane with the hand-off rule; shared by all passes.  Returns true
 // when the lane finished its sample (count and smooth set); a lane still
 // running at hand-off is appended to out_queue instead.
+//
+// Bound by VALU issue.  With run_blocks' scalar lane masks and its cycle test (before:
+// per-lane modes, no test), FP64: the 4096^2 frame at width 1e-4, 4 spp, pass 1
+// 2456 -> 2424 us (2378 without the test) and the whole frame 2969 -> 2915 us; a
+// bounded Julia set, 1400x900, 4 spp 581 -> 145 us; FP32: the set's edge at
+// 1501x1103, 2 spp 742 -> 672 us, the whole set at 2048^2, 4 spp 764 -> 390 us.
 template <class Real, int K, bool kFused>
 __device__ __forceinline__ bool run_lanes(const PipeArgs &a, bool active, Real x, Real y, Real cx,
                                           Real cy, uint i, uint max_iter, Real bsq, double smooth_c,
                                           bool julia, bool blocks, uint tile, uint sample,
                                           Straggler<Real> *out_queue, uint *out_count, uint &count,
                                           double &smooth) {
-    // mode: 0 none, 1 running blocks, 2 pending (checked finish)
-    int mode = !active ? 0 : ((blocks && max_iter - i >= (uint)K) ? 1 : 2);
-    const uint i0 = i;  // iterations the sample had executed before this pass
-    bool replay = false;
-    Real sx = x, sy = y, mx = x, my = y;
-    Real x2 = x * x, y2 = y * y;          // squares of the current state, carried
-    const uint last = max_iter - (uint)K;  // a block may start at i <= last
-    auto block = [&]() {
-        if (mode == 1) {
-            sx = x;
-            sy = y;
-#pragma unroll
-            for (int k = 0; k < K / 2; ++k) cu::quad_step_sq<Real, kFused>(x, y, x2, y2, cx, cy);
-            mx = x;
-            my = y;
-#pragma unroll
-            for (int k = K / 2; k < K; ++k) cu::quad_step_sq<Real, kFused>(x, y, x2, y2, cx, cy);
-            if (x2 + y2 < bsq) {
-                i += K;
-                if (i > last) mode = 2;
-            } else {
-                mode = 2;
-                replay = true;
-            }
-        }
-    };
-    auto keep_going = [&]() {
-        const uint64_t run = cu::ballot(mode == 1);
-        return run != 0 && !(a.handoff && (uint)__popcll(run) <= a.handoff);
-    };
-    // two blocks per trip: the state registers return to place without copies
-    while (keep_going()) {
-        block();
-        if (!keep_going()) break;
-        block();
-    }
+    cu::LaneOrbit<Real> o;
+    o.x = o.sx = o.mx = x;
+    o.y = o.sy = o.my = y;
+    o.cx = cx;
+    o.cy = cy;
+    o.i = i;
+    o.template begin<K>(max_iter, cu::kCycleFirstMixed);
+    uint64_t run = cu::ballot(active && blocks && max_iter - i >= (uint)K);
+    uint64_t failed = 0, ended = cu::ballot(active) & ~run;
+    cu::run_blocks<Real, K, kFused>(o, run, failed, ended, ~0ull, 64u - a.handoff, max_iter, bsq);
     count = 0;
     smooth = 0;
-    if (mode == 2)
-        finish_pending<Real, K, kFused>(x, y, sx, sy, mx, my, cx, cy, i, max_iter, bsq, smooth_c,
-                                        julia, replay, count, smooth);
+    const bool done = cu::in_mask(failed | ended);
+    if (done)
+        finish_sample<Real, K, kFused>(o, failed, max_iter, bsq, smooth_c, julia, count, smooth);
     // this pass's own iterations, whether the sample finished or is handed on
-    const uint64_t executed = mode != 0 ? (uint64_t)(i - i0) : 0u;
+    const uint64_t executed = active ? (uint64_t)(o.i - i) : 0u;
     // lanes still running: append to this wave's sub-queue (one atomic per wave)
-    const bool push = mode == 1;
-    const uint64_t pushers = cu::ballot(push);
-    if (pushers) {
+    if (run) {
         uint base = 0;
-        const uint first = (uint)__ffsll((unsigned long long)pushers) - 1u;
-        if (cu::lane_id() == first) base = atomicAdd(out_count, (uint)__popcll(pushers));
+        const uint first = (uint)__ffsll((unsigned long long)run) - 1u;
+        if (cu::lane_id() == first) base = atomicAdd(out_count, cu::lanes(run));
         base = __shfl(base, (int)first, 64);
-        if (push) {
-            const uint rank = (uint)__popcll(pushers & ((1ull << cu::lane_id()) - 1ull));
+        if (cu::in_mask(run)) {
+            const uint rank = (uint)__popcll(run & ((1ull << cu::lane_id()) - 1ull));
             Straggler<Real> s;
-            s.x = x;
-            s.y = y;
-            s.i = i;
+            s.x = o.x;
+            s.y = o.y;
+            s.i = o.i;
             s.tile = tile;
             s.sample = sample;
             s.pad = 0;
@@ -162,7 +131,7 @@ __device__ __forceinline__ bool run_lanes(const PipeArgs &a, bool active, Real x
         }
     }
     cu::add_iterations(a.iters, executed);
-    return mode == 2;
+    return done;
 }
 
 // Pixel outputs from the in-order sums of its 2^lspp samples: integer mean
@@ -382,11 +351,10 @@ __device__ void drain(const PipeArgs a, const Straggler<Real> *queue, const uint
     const uint lane = cu::lane_id();
     const uint64_t lanes_below = (1ull << lane) - 1ull;
 
-    int mode = 0;  // 0 idle, 1 running unchecked blocks, 2 pending
-    bool replay = false;
-    Real x = 0, y = 0, cx = 0, cy = 0, sx = 0, sy = 0, mx = 0, my = 0, bsq = 4;
-    Real x2 = 0, y2 = 0;  // squares of the current state, carried from step to step
-    uint i = 0, i0 = 0, tile = 0, sample = 0, max_iter = 0;
+    uint64_t run = 0, failed = 0, ended = 0;  // lanes by state (cu::run_blocks); the rest are idle
+    cu::LaneOrbit<Real> o = {};
+    Real bsq = 4;
+    uint i0 = 0, tile = 0, sample = 0, max_iter = 0;
     double smooth_c = 1;
     bool julia = false, blocks = false;
     uint64_t executed = 0;
@@ -405,7 +373,7 @@ __device__ void drain(const PipeArgs a, const Straggler<Real> *queue, const uint
 
     for (;;) {
         // ---- refill idle lanes ----
-        uint64_t idle = cu::ballot(mode == 0);
+        uint64_t idle = ~(run | ended);
         while (idle != 0 && !exhausted) {
             if (cur >= end) {
                 if (next >= last) {
@@ -426,56 +394,37 @@ __device__ void drain(const PipeArgs a, const Straggler<Real> *queue, const uint
             const uint n = (uint)__popcll(idle);
             const uint take = min(n, end - cur);
             const uint rank = (uint)__popcll(idle & lanes_below);
-            if (mode == 0 && rank < take) {
+            const uint64_t taken = idle & cu::ballot(rank < take);
+            bool ok = false;
+            if (cu::in_mask(taken)) {
                 const Straggler<Real> e = queue[(uint64_t)cq * a.subq_capacity + cur + rank];
-                load_straggler<Real>(a, e, x, y, cx, cy, i, tile, sample, max_iter, bsq, smooth_c,
-                                     julia, blocks);
-                i0 = i;
-                replay = false;
-                mode = (blocks && max_iter - i >= (uint)K) ? 1 : 2;
-                x2 = x * x;
-                y2 = y * y;
+                load_straggler<Real>(a, e, o.x, o.y, o.cx, o.cy, o.i, tile, sample, max_iter, bsq,
+                                     smooth_c, julia, blocks);
+                i0 = o.i;
+                o.template begin<K>(max_iter, cu::kCycleFirstMixed);
+                ok = blocks && max_iter - o.i >= (uint)K;
             }
+            const uint64_t can = cu::ballot(ok);
+            run |= can;
+            ended |= taken & ~can;
             cur += take;
-            idle = cu::ballot(mode == 0);
+            idle &= ~taken;
         }
-        if (cu::ballot(mode != 0) == 0) break;
+        if ((run | ended) == 0) break;
 
         // ---- unchecked blocks until enough lanes wait ----
-        for (;;) {
-            if (mode == 1) {
-                sx = x;
-                sy = y;
-#pragma unroll
-                for (int k = 0; k < K / 2; ++k) cu::quad_step_sq<Real, kFused>(x, y, x2, y2, cx, cy);
-                mx = x;
-                my = y;
-#pragma unroll
-                for (int k = K / 2; k < K; ++k) cu::quad_step_sq<Real, kFused>(x, y, x2, y2, cx, cy);
-                if (x2 + y2 < bsq) {
-                    i += K;
-                    if (max_iter - i < (uint)K) mode = 2;
-                } else {
-                    mode = 2;
-                    replay = true;
-                }
-            }
-            const uint64_t run = cu::ballot(mode == 1);
-            const uint waiting = (uint)__popcll(cu::ballot(mode == 2)) +
-                                 (exhausted ? 0u : (uint)__popcll(cu::ballot(mode == 0)));
-            if (run == 0 || waiting >= refill) break;
-        }
+        cu::run_blocks<Real, K, kFused>(o, run, failed, ended, exhausted ? run | ended : ~0ull,
+                                        refill, max_iter, bsq);
 
         // ---- pending lanes finish their sample ----
-        if (mode == 2) {
+        if (cu::in_mask(failed | ended)) {
             uint count;
             double sm;
-            finish_pending<Real, K, kFused>(x, y, sx, sy, mx, my, cx, cy, i, max_iter, bsq,
-                                            smooth_c, julia, replay, count, sm);
-            executed += i - i0;  // the iterations run here; earlier passes counted theirs
+            finish_sample<Real, K, kFused>(o, failed, max_iter, bsq, smooth_c, julia, count, sm);
+            executed += o.i - i0;  // the iterations run here; earlier passes counted theirs
             store_sample(a, tile, sample, count, sm);
-            mode = 0;
         }
+        failed = ended = 0;
     }
     cu::add_iterations(a.iters, executed);
 }

@@ -135,3 +135,26 @@ def test_persistent_kernel(gpu, engine, oracle, steps, chunk, refill, spp, preci
         total += wit
         offset += n
     assert batch.iters.total() == total
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("spp", [1, 4])
+@pytest.mark.parametrize("tune", [(16, 24, 0, 0, 40), (8, 32, 3, 1, 0), (16, 1, 1, 2, 64), (8, 16, 2, 0, 1)])
+def test_frame_pipeline(gpu, engine, oracle, tune, spp, precision):
+    """All views and limits as the tiles of one frame: pass 1, tail passes and drain."""
+    limits = LIMITS + [7, 8, 15, 16, 17, 128, 143, 144, 145, 192, 193]
+    tiles = [tile_of(gpu, v, n, spp, size=(29, 17)) for v in sorted(VIEWS) for n in limits]
+    tiles.append(tile_of(gpu, "home", 300, spp, bailout=3.0))
+    frame = gpu.Frame(engine, tiles, precision)
+    frame.render(gpu.FrameTune(*tune))
+    gpu.synchronize()
+    counts, smooth = frame.counts(), frame.smooth()
+    total, offset = 0, 0
+    for t in tiles:
+        n = t.width * t.height
+        wc, ws, wit = oracle.escape_tile(t, precision)
+        same((counts[offset:offset + n], smooth[offset:offset + n], wit), (wc, ws, wit))
+        total += wit
+        offset += n
+    assert frame.iterations() == total
+    frame.close()

@@ -14,6 +14,8 @@ constexpr uint32_t kMaxPersistentTiles = 1024;  // tile tables staged in LDS
 cu_function function(cu_engine e, const std::string &name);
 void launch(cu_engine e, cu_function f, dim3 grid, dim3 block, void **params, cu_stream s,
             bool timed);
+// 256-thread blocks of `f` that a CU holds at once, by its registers and LDS (asked once)
+uint32_t resident_blocks(cu_function f);
 const char *real_name(int precision);
 bool fused_safe(const cu_tile_desc &t, int precision);
 void validate_tile(const cu_tile_desc &t);

@@ -81,8 +81,6 @@ struct cu_frame_s {
     bool replayed = false;                 // last render was a graph replay (no pass-1 event)
     hipGraph_t graph = nullptr;            // captured render (cu_frame_capture)
     hipGraphExec_t graph_exec = nullptr;
-    cu_function drain_fn = nullptr;        // drain kernel whose occupancy is cached below
-    int drain_blocks_per_cu = 0;           // resident 256-thread drain blocks per CU
 };
 
 namespace cu {
@@ -199,14 +197,7 @@ void enqueue_render(cu_frame f, const cu_frame_tune &tn, const uint32_t *d_palet
         // 256 threads per block: the kernel's queue prefix assumes it.  One
         // resident set of blocks: as many per CU as its registers allow, so every
         // wave slot holds a refilling wave and none waits behind the grid.
-        if (f->drain_fn != drain) {
-            int per_cu = 0;
-            check(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, drain->function, 256, 0),
-                  "hipModuleOccupancyMaxActiveBlocksPerMultiprocessor");
-            f->drain_fn = drain;
-            f->drain_blocks_per_cu = std::max(1, per_cu);
-        }
-        launch(f->engine, drain, dim3(cus * (uint32_t)f->drain_blocks_per_cu), dim3(256), params,
+        launch(f->engine, drain, dim3(cus * resident_blocks(drain)), dim3(256), params,
                stream, false);
     }
     {

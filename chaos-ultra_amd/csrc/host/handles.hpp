@@ -8,6 +8,7 @@
 struct cu_function_s {
     hipFunction_t function;
     std::string name;
+    int resident_blocks = 0;  // 256-thread blocks a CU holds at once (0: not asked yet)
 };
 
 struct cu_module_s {

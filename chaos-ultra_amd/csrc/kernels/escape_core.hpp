@@ -395,9 +395,18 @@ __device__ __forceinline__ void tile_point<float>(const cu_tile_desc &t, uint px
 // Wave-level helpers (wave64).
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 __device__ __forceinline__ uint lane_id() { return __lane_id(); }
-// Lanes in a wave-uniform mask (a scalar; compared as one).
+// Lane 0's value as a scalar (a shuffle would leave it, and every branch on it, per lane).
+__device__ __forceinline__ uint64_t first_lane(uint64_t v) {
+    return ((uint64_t)__builtin_amdgcn_readfirstlane((uint)(v >> 32)) << 32) |
+           __builtin_amdgcn_readfirstlane((uint)v);
+}
+
+// Lanes in a wave-uniform mask, by the scalar instruction: a count the compiler knows
+// to be 64 bits wide it compares in the vector unit.
 __device__ __forceinline__ uint lanes(uint64_t mask) {
-    return (uint)__builtin_amdgcn_readfirstlane(__popcll(mask));
+    uint n;
+    asm("s_bcnt1_i32_b64 %0, %1" : "=s"(n) : "s"(mask) : "scc");
+    return n;
 }
 // The iteration counter is CU_ITER_SLOTS u64 slots; each wave adds its total
 // to one slot chosen by its global wave number, so a launch of a million waves
@@ -462,7 +471,9 @@ __device__ __forceinline__ void run_blocks(LaneOrbit<Real> &o, uint64_t &run, ui
                                            uint64_t &ended, uint64_t counted, uint enough,
                                            uint max_iter, Real bsq) {
     Real x2 = o.x * o.x, y2 = o.y * o.y;  // squares of the current state, carried
-    while (run != 0 && lanes(counted & ~run) < enough) {
+    enough = min(enough, lanes(counted));  // with no lane running, all counted ones wait
+    if (lanes(counted & ~run) >= enough) return;
+    for (;;) {
         uint64_t inside, due, again;
         do {
             if (in_mask(run)) {
@@ -497,6 +508,7 @@ __device__ __forceinline__ void run_blocks(LaneOrbit<Real> &o, uint64_t &run, ui
                 o.until = min(next_hold<K>(o.i), max_iter - (uint)K + 1u);
             }
         }
+        if (lanes(counted & ~run) >= enough) return;
     }
 }
 

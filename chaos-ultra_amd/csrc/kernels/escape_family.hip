@@ -155,14 +155,18 @@ __device__ void escape_tile_samples(const cu_tile_desc &t, double smooth_c, uint
 // the exact escape step in the half of their last block that holds it
 // (cu::locate_escape), finish their sample, start the next sample of the same
 // pixel or write the pixel, and idle lanes take new pixels from a wave-private
-// chunk of the global pixel queue (one atomic per `chunk` pixels).  Pixels of
+// chunk of the global pixel queue (one atomic per at most `chunk` pixels).  Pixels of
 // one tile are numbered row-major from the tile's work_offset.  There is no
 // barrier after the tile table is staged, and every wave leaves once the queue
 // is exhausted and its lanes are idle.
 //
-// Bound by VALU issue, then by the longest orbits at the end.  Batches of 32 and 24
-// uneven tiles, FP64, tune 32/32/256/16: 7.7 -> 3.0 and 10.0 -> 2.8 ms with the cycle
-// test (1.8e10 and 2.3e10 loop iterations); 32 tiles in FP32 9.4 -> 1.9 ms.
+// Bound by VALU issue, then by the longest orbits at the end (a lone wave takes about
+// 17 ns a step, so 65536 of them 1.1 ms).  Batches of 32 and 24 uneven tiles, FP64,
+// tune 32/32/256/16: 7.7 -> 2.8 and 10.0 -> 2.2 ms (1.8e10 and 2.3e10 loop iterations)
+// with the cycle test, scalar lane masks and cursor (106 VGPRs against 115 with a
+// cursor the compiler kept per lane) and one resident set of waves; 32 tiles in FP32
+// 9.4 -> 1.8 ms.  Giving waves with old orbits issue priority (s_setprio) made no
+// batch faster and frames' tails up to 8 % slower.
 template <class Real, int K, bool kFused>
 __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, uint n_tiles,
                                         uint64_t total, uint *counts, double *smooth,
@@ -188,34 +192,49 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
     uint max_iter = 0;
     uint64_t executed = 0;
 
-    // Wave-uniform chunk cursor.  A wave's first chunk follows from its number,
-    // so the launch does not start with every wave's atomic on the one counter;
-    // the counter hands out the chunks after all of the first ones.
+    // Wave-uniform chunk cursor.  A wave's first items follow from its number, so the
+    // launch does not start with every wave's atomic on the one counter; the counter
+    // hands out the items after all of the first ones.  A grab takes `chunk` items
+    // while that is at most half of what the launch's waves would each get of the
+    // rest, and fewer towards the end (down to a lane's worth each): one wave's last
+    // 256 pixels of deep orbits would outlast every other wave.
     const uint64_t wave_global = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) +
                                                                 (threadIdx.x >> 6));
-    const uint64_t first_items = (uint64_t)gridDim.x * (blockDim.x >> 6) * chunk;
-    uint64_t cur = wave_global * chunk;
-    uint64_t end = min(cur + chunk, total);
+    const uint waves = gridDim.x * (blockDim.x >> 6);
+    const uint share = 33u - __clz(waves);  // log2 of at least twice the waves
+    auto grab_size = [&](uint64_t rest) {
+        const uint64_t part = rest >> share;
+        const uint least = min(chunk, 64u);
+        return part >= chunk ? chunk : max((uint)part, least);
+    };
+    const uint first = grab_size(total);
+    const uint64_t first_items = (uint64_t)waves * first;
+    // `left` of the items from `cur` on are this wave's; scalars, so that the branches
+    // on them leave the lane masks scalar too.
+    uint64_t cur = wave_global * first;
+    auto items_from = [&](uint64_t at, uint size) {
+        const uint n = at < total ? (uint)min((uint64_t)size, total - at) : 0u;
+        return (uint)__builtin_amdgcn_readfirstlane(n);
+    };
+    uint left = items_from(cur, first);
     bool exhausted = false;
 
     for (;;) {
         // ---- refill idle lanes ----
         uint64_t idle = ~(run | ended);
         while (idle != 0 && !exhausted) {
-            if (cur >= end) {
+            if (left == 0) {
+                const uint size = grab_size(cur < total ? total - cur : 0u);
                 unsigned long long base = 0;
-                if (lane == 0 && first_items < total) base = atomicAdd(queue, (unsigned long long)chunk);
-                base = first_items + __shfl(base, 0, 64);
-                if (base >= total) {
+                if (lane == 0 && first_items < total) base = atomicAdd(queue, (unsigned long long)size);
+                cur = first_items + cu::first_lane(base);
+                left = items_from(cur, size);
+                if (left == 0) {
                     exhausted = true;
                     break;
                 }
-                cur = base;
-                end = min((uint64_t)base + chunk, total);
             }
-            const uint n = (uint)__popcll(idle);
-            const uint64_t avail = end - cur;
-            const uint take = (uint)min((uint64_t)n, avail);
+            const uint take = min(cu::lanes(idle), left);
             const uint rank = (uint)__popcll(idle & lanes_below);
             const uint64_t taken = idle & cu::ballot(rank < take);
             bool blocks = false;
@@ -246,6 +265,7 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
             run |= ok;
             ended |= taken & ~ok;
             cur += take;
+            left -= take;
             idle &= ~taken;
         }
         if ((run | ended) == 0) break;

@@ -186,7 +186,8 @@ int cu_renderer_supply_default_values(cu_renderer r, cu_rendering_model *model, 
 int cu_renderer_read_output(cu_renderer r, uint32_t *rgba, size_t count);
 /* Iterations executed by the renderer's fractal module since it was loaded: the
  * sum of its cu_iteration_slots (each sample adds the loop bodies computeFractal
- * ran — the escape step, or maxIterations for an orbit that never escapes).  The
+ * runs — the escape step, or maxIterations for an orbit that never escapes, also
+ * where that is known earlier because its state has come back).  The
  * reference has no counterpart; a caller takes differences around a render to
  * get its Giga-iterations/s. */
 int cu_renderer_iterations(cu_renderer r, unsigned long long *total);
@@ -272,8 +273,8 @@ int cu_tile_init(cu_tile_desc *tile, double lbx, double lby, double rtx, double 
 /* Tuning of the persistent launch (chosen by the autotuner). */
 typedef struct cu_tune {
     uint32_t block_steps;   /* K: unchecked iterations per block (8, 16, 32)       */
-    uint32_t waves_per_cu;  /* resident waves per CU in the persistent grid         */
-    uint32_t chunk;         /* pixels taken per global-queue grab                    */
+    uint32_t waves_per_cu;  /* waves per CU in the persistent grid (at most what fits at once) */
+    uint32_t chunk;         /* pixels taken per global-queue grab, fewer near its end */
     uint32_t refill_lanes;  /* retire/refill when at least this many lanes are idle  */
 } cu_tune;
 
@@ -291,7 +292,8 @@ int cu_engine_destroy(cu_engine e);
  * inputs can reach that range; see cu_tile_fused_safe). */
 int cu_tile_fused_safe(const cu_tile_desc *tile, int precision, int *safe);
 
-/* Iterations executed (an interior sample counts max_iter) are accumulated in
+/* Iterations executed (an interior sample counts max_iter, also where its orbit
+ * has become a cycle of states before that and is not run on) are accumulated in
  * CU_ITER_SLOTS device u64 slots: each wave adds to one slot, the total is the
  * sum of the slots (cu_iters_total). */
 #define CU_ITER_SLOTS 1024u

@@ -21,8 +21,7 @@ extern "C" __global__ __launch_bounds__(64) void referenceOrbitDouble(
 // it can go through the scalar cache.  The second bound (8 waves per SIMD)
 // keeps the kernels within 64 VGPRs, so that a CU's 32 wave slots can all be
 // filled; without it the compiler keeps a whole block's orbit reads in flight.
-// Blocks of 32 steps: against 16, 7-9 % faster at 1e-10 and 1e-20 and the same at
-// 1e-6, where a rebase reruns more of a longer block.  Block shapes: perturb_frame.
+// Blocks of 32 steps.  Block shapes: perturb_frame.
 extern "C" __global__ __launch_bounds__(256, 8) void perturbFloat(
     DeepArgs a, const OrbitEntry<float> *__restrict__ orbit) {
     perturb_frame<float, 32, 2, 2, 20u * 1024u>(a, orbit);

@@ -24,12 +24,12 @@
 // Pauldelbrot's test |z|^2 < eps |Z|^2 marks a pixel glitched and the host
 // re-renders glitched pixels around a secondary reference.
 //
-// Hot loop: unchecked blocks of K steps (one orbit load and 8 FMA-class
-// VALU ops per step).  A block ends early at the first step where some lane's
-// rebase test fires, and those lanes take the rebase there; escape is tested
-// once, at the block's end (escape is permanent for bailout_sq >= 4, |c| <= 2),
-// and only a block with an escape is replayed with checked steps — the same
-// operation sequence as the oracle's checked loop.
+// Hot loop: blocks of K steps (one orbit load and 9 VALU ops per step).  Where all
+// lanes of a wave stand at the same orbit entry and none rebases, the entries come
+// through the scalar cache; otherwise each lane reads its own and takes its rebases
+// inside the block.  Escape is tested once, at the block's end (escape is permanent
+// for bailout_sq >= 4, |c| <= 2), and the blocks with an escape are replayed, all
+// lanes' together, with checked steps — the oracle's operation sequence.
 #pragma once
 #include "cu_types.hpp"
 #include "escape_core.hpp"
@@ -185,6 +185,24 @@ __device__ __forceinline__ bool rebase_test(Real Zx, Real Zy, Real h, Real dx, R
     return cu::fma_r(Zx, dx, Zy * dy) < -h;
 }
 
+// The delta of an earlier rebase, for the cycle test.  After a rebase the reference
+// index is 0, so the pixel's future is a function of its delta alone: a delta that
+// comes back makes the orbit a cycle that never escapes, and the checked loop's result
+// is the one at max_iter.  (-0 compares equal to 0: a zero's sign changes no later
+// magnitude.)  Before the first rebase the pixel's start is held, a delta of 0 at index
+// 0.  Pixels of the set's interior rebase every few hundred steps; by a count on the CPU
+// (1e-6 frame, maxIter 50000, three quarters interior) the test leaves 0.48 of the steps
+// with FP64 deltas and 0.28 with FP32 ones.
+template <class Real>
+struct HeldDelta {
+    Real x = 0, y = 0;
+    __device__ __forceinline__ bool is(Real dx, Real dy) const { return dx == x && dy == y; }
+    __device__ __forceinline__ void take(Real dx, Real dy) {
+        x = dx;
+        y = dy;
+    }
+};
+
 // One checked step of the perturbation loop (the oracle's or_perturb_pixel
 // body).  Returns 0 to continue, 1 escaped (mag set), 2 max_iter, 3 glitched.
 template <class Real>
@@ -251,23 +269,41 @@ __device__ __forceinline__ uint64_t unchecked_block(Ptr zp, Real &dx, Real &dy, 
     return flagged;
 }
 
-// The same steps, stopping at the first step k0 at which some lane's rebase test
-// fires: every lane is left in its state at step k0, `fired` holds the lanes whose
-// test fired there and `end` is orbit entry zp[k0].  Returns k0 (K, with `end`
-// = zp[K], when no test fires).  Only lanes in `running` count.  Its branches keep
-// the orbit reads from being issued ahead, so it runs after unchecked_block
-// reported a firing, or directly while rebases come in consecutive blocks.
-template <class Real, int K, class Ptr>
-__device__ __forceinline__ uint stopping_block(Ptr zp, Real &dx, Real &dy, Real dcx, Real dcy,
-                                               uint64_t running, uint64_t &fired,
-                                               OrbitEntry<Real> &end) {
+// K steps in which each lane takes its own rebases: lane's index is m at step 0, and
+// a lane whose test fires (or, kEnd, whose index is M) restarts the reference there
+// with d = z and takes the step from Z_0 = 0, as the checked loop does, while the
+// others go on.  So a step costs what an unchecked one does, plus a branch and, where
+// some lane rebases, a few masked instructions; entries come one step ahead of their
+// use, and a rebased lane's next one is Z_1, the same for all.  Every read lies in
+// [0, m + K], clamped to M with kEnd.  Returns the running lanes that rebased, with the delta of
+// each one's last rebase in (rx, ry); `end` is the entry at the final index.
+template <class Real, int K, bool kEnd, class Ptr>
+__device__ __forceinline__ uint64_t rebasing_block(Ptr orbit, uint M, const OrbitEntry<Real> &z1,
+                                                   uint64_t running, uint &m, Real &dx, Real &dy,
+                                                   Real dcx, Real dcy, Real &rx, Real &ry,
+                                                   OrbitEntry<Real> &end) {
+    uint64_t rebased = 0;
+    int first = (int)m;  // the lane's index at step k is first + k
+    OrbitEntry<Real> e = load_entry<Real>(orbit + first);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const OrbitEntry<Real> e = load_entry<Real>(zp + k);
-        fired = cu::ballot(rebase_test(e.x, e.y, e.h, dx, dy)) & running;
-        if (fired != 0) {
-            end = e;
-            return (uint)k;
+        int ahead = first + (k + 1);
+        if constexpr (kEnd) ahead = min(ahead, (int)M);
+        OrbitEntry<Real> next = load_entry<Real>(orbit + ahead);
+        bool fire = rebase_test(e.x, e.y, e.h, dx, dy);
+        if constexpr (kEnd) fire = fire || first + k == (int)M;
+        const uint64_t firing = cu::ballot(fire) & running;
+        if (firing != 0) {
+            cu::seldom();
+            rebased |= firing;
+            if (cu::in_mask(firing)) {
+                dx = rx = e.x + dx;
+                dy = ry = e.y + dy;
+                e.x = 0;
+                e.y = 0;
+                next = z1;
+                first = -k;
+            }
         }
         const Real ax = cu::fma_r((Real)2, e.x, dx);
         const Real ay = cu::fma_r((Real)2, e.y, dy);
@@ -275,116 +311,129 @@ __device__ __forceinline__ uint stopping_block(Ptr zp, Real &dx, Real &dy, Real 
         const Real ndy = cu::fma_r(ax, dy, cu::fma_r(ay, dx, dcy));
         dx = ndx;
         dy = ndy;
+        e = next;
     }
-    end = load_entry<Real>(zp + K);
-    return (uint)K;
+    m = (uint)(first + K);
+    end = e;
+    return rebased;
 }
 
 // Whole pixel; lanes whose `active` is false only take part in the ballots.
 //
-// While every running lane can take an unchecked block (its iteration budget and
-// the orbit both have K steps left), the whole wave takes one, in wave-uniform
-// control flow: lanes that have finished compute along with their m held at 0,
-// so every read stays in bounds, and change nothing (ballots are masked to the
-// running lanes).  When the running lanes all read the same orbit entries (same
-// m), the block reads them through the scalar cache; otherwise each lane reads
-// its own entries from the LDS copy, or from global memory past it.  When some
-// running lane cannot take a block, every running lane takes one checked step.
+// With rebasing, the running lanes take blocks of K steps together, so their
+// iteration count n is one scalar.  While they all read the same orbit entries (same
+// m) a block reads them through the scalar cache and only collects whether a rebase
+// test fired; if one did, it is run again as a rebasing_block, which is taken at once
+// where lanes stand at different entries or the last two blocks had to be rerun.
+// Escape is tested at a block's end (it is permanent for bailout_sq >= 4, |c| <= 2):
+// a lane that left inside a block keeps that block's start, and when no lane runs any
+// more all such lanes replay theirs together with checked steps, the oracle's loop
+// body; the last max_iter % K steps are checked ones too.  A lane whose rebase delta
+// has come back is at a cycle's end (HeldDelta).
 //
-// A block ends at step k0 for the whole wave: K, or the first step at which a
-// running lane's rebase test fired (found by rerunning the block in the form that
-// stops there, or by running that form directly after two blocks that stopped).
-// There the escape test runs on z = Z_m + d.  Escaped (at step k0, hence at some
-// step of the block since escape is permanent): the lane replays the block with
-// checked steps from its start.  Otherwise the lanes whose test fired take the
-// rebase d = z, m = 0 with n counting the k0 steps taken, and the others simply
-// stand at step k0.  The checked loop would take the same rebase at the same
-// state and then step from Z_0 = 0; the next block starts there, and its first
-// rebase test, at m = 0 with Z_0 = 0 and |Z_0|^2 = 0, compares a zero with -0
-// and does not fire, while lanes that did not fire repeat a test that passed —
-// so every block advances.
+// Without rebasing every step is a checked one (the glitch test needs each).
+//
+// Bound by VALU issue; 1920x1080, without the reference orbit's time, FP32 / FP64
+// deltas: 1e-10 (each pixel rebases on its own) 1.50 / 2.24 -> 1.09 / 1.92 ms, a
+// shallow frame of width 1 2.85 / 3.80 -> 0.70 / 1.15 ms, 1e-20 (few rebases) 1.20 / 2.03
+// -> 1.16 / 1.94 ms; before, a block stopped for the whole wave at its first rebase,
+// and each escape was replayed as it came, 32 checked steps for one lane.  1e-6, three
+// quarters interior, 18.7 / 32.7 -> 8.9 / 19.3 ms, 11.0 / 22.0 of it by the cycle test.
 template <class Real, int K>
 __device__ int perturb_pixel(const OrbitView<Real> &Z, uint M, Real dcx, Real dcy, uint max_iter,
                              Real bsq, bool rebase, Real geps, bool active, uint &n_out,
                              Real &mag_out) {
     Real dx = 0, dy = 0;
-    uint m = 0, n = 0;
+    uint m = 0, n_lane = 0;
     int state = active ? 0 : 4;
     mag_out = 0;
-    uint streak = 0;  // wave-uniform: consecutive blocks that stopped at a rebase
-    for (;;) {
-        const uint64_t running = cu::ballot(state == 0);
-        if (running == 0) break;
-        const bool can = rebase && max_iter - n >= (uint)K && M - m >= (uint)K;
-        const bool block = (cu::ballot(can) & running) == running;
-        bool replay = false;
-        if (block) {
-            const Real sx = dx, sy = dy;
-            const uint mu = __builtin_amdgcn_readlane(m, (int)__builtin_ctzll(running));
-            const bool same = (cu::ballot(m != mu) & running) == 0;
-            const bool lds = (cu::ballot(m + (uint)K >= Z.staged) & running) == 0;
+    if (rebase) {
+        uint64_t run = cu::ballot(active), failed = 0;
+        uint n = 0;                      // iterations of the running lanes
+        Real sx = 0, sy = 0;             // block start
+        uint sm = 0;
+        Real rx = 0, ry = 0;             // delta of the lane's last rebase
+        HeldDelta<Real> held;
+        uint hold = 0;                   // iteration count from which the next one is held
+        uint streak = 0;                 // consecutive blocks rerun for a rebase
+        const OrbitEntry<Real> z1 = load_entry<Real>(Z.global + min(1u, M));
+        while (run != 0 && max_iter - n >= (uint)K) {
+            if (cu::in_mask(run)) {
+                sx = dx;
+                sy = dy;
+                sm = m;
+            } else {
+                m = 0;  // lanes that do not run compute along from entry 0, for no effect
+            }
+            const uint mu = __builtin_amdgcn_readlane(m, (int)__builtin_ctzll(run));
+            const bool same = (cu::ballot(m != mu) & run) == 0;
+            const bool near = (cu::ballot(M - m < (uint)K) & run) != 0;
             OrbitEntry<Real> e;
-            uint64_t fired = 0;
-            uint k0 = K;
-            // after two blocks in a row that stopped at a rebase, rebases come often
-            // here: go straight to the form that stops at the first one
-            bool stop = streak >= 2;
-            if (!stop) {
-                uint64_t flagged;
-                if (same) {
+            uint64_t rebased = 0;
+            bool plain = same && !near && streak < 2;
+            if (plain) {
+                const Real bx = dx, by = dy;
+                plain = (unchecked_block<Real, K>(Z.global + mu, dx, dy, dcx, dcy) & run) == 0;
+                if (plain) {
                     e = load_entry<Real>(Z.global + (mu + (uint)K));
-                    flagged = unchecked_block<Real, K>(Z.global + mu, dx, dy, dcx, dcy);
-                } else if (lds) {
-                    e = load_entry<Real>(Z.lds + (m + (uint)K));
-                    flagged = unchecked_block<Real, K>(Z.lds + m, dx, dy, dcx, dcy);
+                    m += (uint)K;
+                    streak = 0;
                 } else {
-                    e = load_entry<Real>(Z.global + (m + (uint)K));
-                    flagged = unchecked_block<Real, K>(Z.global + m, dx, dy, dcx, dcy);
-                }
-                if ((flagged & running) != 0) {  // a rebase test fired: rerun up to there
-                    dx = sx;
-                    dy = sy;
-                    stop = true;
+                    dx = bx;
+                    dy = by;
+                    ++streak;
                 }
             }
-            if (stop) {
-                if (same)
-                    k0 = stopping_block<Real, K>(Z.global + mu, dx, dy, dcx, dcy, running, fired, e);
-                else if (lds)
-                    k0 = stopping_block<Real, K>(Z.lds + m, dx, dy, dcx, dcy, running, fired, e);
+            if (!plain) {
+                if (near)
+                    rebased = rebasing_block<Real, K, true>(Z.global, M, z1, run, m, dx, dy, dcx,
+                                                            dcy, rx, ry, e);
+                else if ((cu::ballot(m + (uint)K >= Z.staged) & run) == 0)
+                    rebased = rebasing_block<Real, K, false>(Z.lds, M, z1, run, m, dx, dy, dcx,
+                                                             dcy, rx, ry, e);
                 else
-                    k0 = stopping_block<Real, K>(Z.global + m, dx, dy, dcx, dcy, running, fired,
-                                                 e);
+                    rebased = rebasing_block<Real, K, false>(Z.global, M, z1, run, m, dx, dy, dcx,
+                                                             dcy, rx, ry, e);
+                if (rebased == 0) streak = 0;
             }
-            streak = k0 < (uint)K ? streak + 1 : 0;
-            if (state == 0) {
-                const Real zx = e.x + dx;
-                const Real zy = e.y + dy;
-                const Real mag = cu::fma_r(zx, zx, zy * zy);
-                if (!(mag < bsq)) {
-                    dx = sx;
-                    dy = sy;
-                    replay = true;
-                } else {
-                    n += k0;
-                    m += k0;
-                    if (cu::in_mask(fired)) {
-                        dx = zx;
-                        dy = zy;
-                        m = 0;
-                    }
+            const Real zx = e.x + dx;
+            const Real zy = e.y + dy;
+            const uint64_t out = run & ~cu::ballot(cu::fma_r(zx, zx, zy * zy) < bsq);
+            if (out != 0) {
+                cu::seldom();
+                failed |= out;
+                run &= ~out;
+                if (cu::in_mask(out)) n_lane = n;  // where its block starts
+            }
+            n += (uint)K;
+            rebased &= run;
+            if (rebased != 0) {
+                cu::seldom();
+                const uint64_t cycle = rebased & cu::ballot(held.is(rx, ry));
+                if (cu::in_mask(cycle)) {
+                    n_lane = max_iter;
+                    state = 2;
                 }
+                run &= ~cycle;
+            }
+            if (n >= hold) {
+                cu::seldom();
+                held.take(rx, ry);
+                hold = n + n / 2;
             }
         }
-        if (state == 0 && (!block || replay)) {
-            const int steps = block ? K : 1;
-            for (int s = 0; s < steps && state == 0; ++s)
-                state = checked_step<Real>(Z, M, dx, dy, m, n, dcx, dcy, max_iter, bsq, rebase,
-                                           geps, mag_out);
-            if (state != 0) m = 0;  // finished: later blocks read from entry 0
+        if (cu::in_mask(run)) n_lane = n;
+        if (cu::in_mask(failed)) {
+            dx = sx;
+            dy = sy;
+            m = sm;
         }
     }
-    n_out = n;
+    while (cu::ballot(state == 0) != 0)
+        if (state == 0)
+            state = checked_step<Real>(Z, M, dx, dy, m, n_lane, dcx, dcy, max_iter, bsq, rebase,
+                                       geps, mag_out);
+    n_out = n_lane;
     return state;
 }
 

@@ -158,3 +158,16 @@ def test_frame_pipeline(gpu, engine, oracle, tune, spp, precision):
         offset += n
     assert frame.iterations() == total
     frame.close()
+
+
+# (centre, width, limit): a reference that escapes early so that every interior pixel
+# rebases, one inside the set, one of a few steps (checked steps only), a shallow frame
+@pytest.mark.parametrize("centre,width,limit", [
+    ((-0.743643887037151, 0.131825904205330), 1e-6, 30000),
+    ((-0.743643887037151 + 4e-8, 0.131825904205330 - 6e-8), 1e-6, 30000),
+    ((0.5, 0.0), 1e-3, 3000), ((0.26, 1e-3), 0.05, 4000), ((-0.25, 0.125), 1.0, 2000),
+    ((-1.0, 0.0), 0.5, 700), ((0.0, 0.0), 0.5, 97)])
+@pytest.mark.parametrize("method", [32, 64])
+def test_perturbation(gpu, engine, oracle, centre, width, limit, method):
+    """Rebased deltas that come back end the pixel with the checked loop's result."""
+    deep_case(gpu, engine, oracle, gpu.make_deep(*centre, width, 45, 27, limit, 256.0), method)

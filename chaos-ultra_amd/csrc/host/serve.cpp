@@ -306,7 +306,7 @@ void dispatch(cu_serve_s *s, Session &ss, Slot &sl, const Request &rq) {
         uint64_t n = (uint64_t)W * H;
         void *out = sl.d_sum;
         void *params[] = {&p, &n, &out};
-        const unsigned blocks = (unsigned)std::min<uint64_t>((n + 255) / 256, 2048);
+        const unsigned blocks = (unsigned)std::min<uint64_t>((n + 1023) / 1024, 512);
         launch(s->engine, s->checksum, dim3(blocks), dim3(256), params, &sl.wrap, false);
     }
     check(hipMemcpyAsync(sl.h_sum, sl.d_sum, 8, hipMemcpyDeviceToHost, st), "hipMemcpyAsync");

@@ -366,15 +366,27 @@ extern "C" __global__ __launch_bounds__(256) void composeSmooth(
 }
 
 // Order-sensitive checksum of n words: sum of p[i] * (2i + 1) mod 2^64, added to
-// *out (integer addition, so the result does not depend on the schedule).
+// *out (integer addition, so the result does not depend on the schedule).  p is
+// 16-byte aligned (an allocation's start).  All blocks add to one address, about 10 ns
+// each: with an atomic per wave of 2048 blocks a 1280x720 image took 100-115 us, with
+// one per block of at most 512 and four words per load it takes 8.5 us.
 extern "C" __global__ __launch_bounds__(256) void checksumU32(const uint *p, uint64_t n,
                                                               unsigned long long *out) {
+    __shared__ unsigned long long part[4];
+    const uint4 *q = reinterpret_cast<const uint4 *>(p);
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint64_t acc = 0;
-    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
-         k += (uint64_t)gridDim.x * blockDim.x)
-        acc += (uint64_t)p[k] * (2ull * k + 1ull);
+    for (uint64_t k = first; k < n / 4; k += (uint64_t)gridDim.x * blockDim.x) {
+        const uint4 v = q[k];
+        const uint64_t w = 8ull * k + 1ull;
+        acc += v.x * w + v.y * (w + 2ull) + v.z * (w + 4ull) + v.w * (w + 6ull);
+    }
+    const uint64_t last = n / 4 * 4 + first;  // the words after the last whole four
+    if (last < n) acc += (uint64_t)p[last] * (2ull * last + 1ull);
     acc = __ockl_wfred_add_u64(acc);
-    if (cu::lane_id() == 0 && acc) atomicAdd(out, (unsigned long long)acc);
+    if (cu::lane_id() == 0) part[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(out, part[0] + part[1] + part[2] + part[3]);
 }
 
 extern "C" __global__ __launch_bounds__(256) void fillU32(uint *p, uint value, uint64_t n) {

@@ -21,7 +21,7 @@ import time
 
 import numpy as np
 
-from . import abi
+from . import _read_back, abi
 from .abi import FrameDone, FrameRequest, ServeConfig, ServeReport
 
 RESOLUTIONS = ((1280, 720), (1920, 1080), (3840, 2160))
@@ -69,7 +69,7 @@ class Server:
         return buf.value.decode()
 
     def read_rgba(self, session: int, width: int, height: int) -> np.ndarray:
-        out = np.empty(width * height, np.uint32)
+        out = _read_back.empty(width * height, np.uint32)
         abi.call("cu_serve_read_rgba", self.handle, session, out.ctypes.data_as(C.c_void_p), out.size)
         return out.reshape(height, width)
 

@@ -250,7 +250,8 @@ int cu_deep_create(cu_engine e, const cu_deep_desc *desc, int method, cu_deep *o
         d->d_smooth = device_alloc(pixels * 8);
         d->d_glitch = device_alloc(pixels);
         d->d_iters = device_alloc(CU_ITER_SLOTS * 8);
-        for (hipEvent_t &ev : d->ev) check(hipEventCreate(&ev), "hipEventCreate");
+        for (int k = 0; k < 3; ++k) d->ev[k] = mark_event();
+        check(hipEventCreate(&d->ev[3]), "hipEventCreate");
         *out = d;
     });
     if (rc != CU_OK && d) free_deep(d);

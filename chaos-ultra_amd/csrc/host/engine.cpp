@@ -35,6 +35,12 @@ void launch(cu_engine e, cu_function f, dim3 grid, dim3 block, void **params, cu
     }
 }
 
+hipEvent_t mark_event() {
+    hipEvent_t ev = nullptr;
+    check(hipEventCreateWithFlags(&ev, hipEventDisableSystemFence), "hipEventCreateWithFlags");
+    return ev;
+}
+
 uint32_t resident_blocks(cu_function f) {
     if (f->resident_blocks == 0) {
         int per_cu = 0;
@@ -212,7 +218,7 @@ int cu_engine_create(const char *dir, cu_engine *out) {
         if (rc != CU_OK) fail(rc, cu_last_error());
         auto *e = new cu_engine_s();
         e->module = m;
-        check(hipEventCreate(&e->start), "hipEventCreate");
+        e->start = mark_event();
         check(hipEventCreate(&e->stop), "hipEventCreate");
         *out = e;
     });
@@ -289,7 +295,7 @@ int cu_escape_tiles_persistent_capture(cu_engine e, int precision, int variant,
         std::lock_guard<std::mutex> lock(e->mutex);
         ensure_device();
         g = new cu_graph_s();
-        check(hipEventCreate(&g->start), "hipEventCreate");
+        g->start = mark_event();
         check(hipEventCreate(&g->stop), "hipEventCreate");
         hipStream_t cs = nullptr;
         check(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking), "hipStreamCreateWithFlags");

@@ -294,8 +294,8 @@ int cu_frame_create(cu_engine e, const cu_tile_desc *tiles, uint32_t n_tiles, in
                         hipMemcpyHostToDevice), "hipMemcpy H2D");
         check(hipMemcpy(f->d_smooth_c, smooth_c.data(), smooth_c.size() * 8,
                         hipMemcpyHostToDevice), "hipMemcpy H2D");
-        check(hipEventCreate(&f->ev_start), "hipEventCreate");
-        check(hipEventCreate(&f->ev_pass1), "hipEventCreate");
+        f->ev_start = mark_event();
+        f->ev_pass1 = mark_event();
         check(hipEventCreate(&f->ev_end), "hipEventCreate");
         *out = f;
     });

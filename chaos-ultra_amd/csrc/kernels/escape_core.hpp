@@ -64,21 +64,6 @@ __device__ __forceinline__ void quad_step_sq(Real &x, Real &y, Real &x2, Real &y
     y2 = y * y;
 }
 
-// Where the replay of a failed block starts: at its midpoint (iteration
-// i + half) when that state is still inside, else at its start.
-template <class Real>
-__device__ __forceinline__ void replay_start(Real &x, Real &y, uint &i, Real sx, Real sy, Real mx,
-                                             Real my, Real bailout_sq, uint half) {
-    if (mx * mx + my * my < bailout_sq) {
-        x = mx;
-        y = my;
-        i += half;
-    } else {
-        x = sx;
-        y = sy;
-    }
-}
-
 // Checked steps from (x, y, i) until the bailout test fails or i reaches
 // max_iter: the reference loop, for lanes that cannot use an unchecked block.
 template <class Real, bool kFused>
@@ -174,96 +159,6 @@ __device__ __forceinline__ void seldom() { asm volatile(""); }
 template <int K>
 __device__ __forceinline__ uint next_hold(uint i) {
     return i + ((i / 2 + (uint)K - 1u) & ~((uint)K - 1u));
-}
-
-// The reference loop  while (i < maxIter && x*x+y*y < R^2) { step; ++i; }
-// with unchecked blocks of K steps when `blocks` holds (escape is permanent for
-// these inputs) and a checked tail/replay.
-//
-// From kCycleFirst iterations on, each block that ends inside also compares its
-// end state with a held earlier one.  A step is a function of the state alone, so
-// a state that comes back makes the orbit a cycle of states that have all passed
-// the bailout test or lie between two block ends that did (escape is permanent):
-// it never escapes, and the loop's result is the one at maxIter.  (The comparison
-// takes -0 for 0; a zero's sign never changes a magnitude of later states.)  Most
-// interior orbits become such cycles long before maxIter: the attracting cycle is
-// reached to the last bit.  What bounds the kernels is VALU issue, 104 FP64
-// instructions per 16-step block; the test adds one compare to a block (the
-// second one only where the first holds), and none below kCycleFirst.  max_iter
-// and `blocks` are the same for all active lanes (one tile per launch).
-template <class Real, int K, bool kFused>
-__device__ __forceinline__ Orbit<Real> escape_orbit(Real x, Real y, Real cx, Real cy,
-                                                     uint max_iter, Real bailout_sq,
-                                                     bool blocks) {
-    uint i = 0;
-    if (blocks) {
-        Real sx, sy, mx, my;
-        auto block = [&]() {  // whether the orbit is still inside after K steps
-            sx = x;
-            sy = y;
-#pragma unroll
-            for (int k = 0; k < K / 2; ++k) quad_step<Real, kFused>(x, y, cx, cy);
-            mx = x;
-            my = y;
-#pragma unroll
-            for (int k = K / 2; k < K; ++k) quad_step<Real, kFused>(x, y, cx, cy);
-            return x * x + y * y < bailout_sq;
-        };
-        bool inside = true;
-        while (i < kCycleFirst && max_iter - i >= (uint)K) {
-            inside = block();
-            if (!inside) break;
-            i += K;
-        }
-        if (inside) {
-            // the lanes here have all run the same number of iterations, j: a scalar
-            uint j = __builtin_amdgcn_readfirstlane(i), hold = next_hold<K>(j);
-            Real hx = x, hy = y;
-            while (max_iter - j >= (uint)K) {
-                inside = block();
-                if (!inside) break;
-                j += K;
-                if (__ballot(y == hy) != 0) {
-                    seldom();
-                    if (y == hy && x == hx) {
-                        j = max_iter;
-                        break;
-                    }
-                }
-                if (j >= hold) {
-                    seldom();
-                    hx = x;
-                    hy = y;
-                    hold = next_hold<K>(j);
-                }
-            }
-            i = j;
-        }
-        if (!inside) replay_start(x, y, i, sx, sy, mx, my, bailout_sq, (uint)K / 2);
-    }
-    Orbit<Real> r;
-    r.escaped = false;
-    r.mag2 = 0;
-    while (i < max_iter) {
-        const Real x2 = x * x;
-        const Real y2 = y * y;
-        const Real m = x2 + y2;
-        if (!(m < bailout_sq)) {
-            r.escaped = true;
-            r.mag2 = m;
-            break;
-        }
-        const Real xn = (x2 - y2) + cx;
-        if constexpr (kFused) {
-            y = fma_r(x * y, (Real)2, cy);
-        } else {
-            y = ((x + x) * y) + cy;
-        }
-        x = xn;
-        ++i;
-    }
-    r.n = i;
-    return r;
 }
 
 // Whether unchecked blocks are valid: R >= 2 and, when c is fixed (Julia), |c| <= R.
@@ -461,8 +356,17 @@ struct LaneOrbit {
 // `enough` of the `counted` lanes do not.  Which lanes run is wave-uniform: a lane
 // leaves `run` for `failed` when its block ends outside (the escape lies in that
 // block), or for `ended` when fewer than K of its max_iter steps are left or, with i
-// set to max_iter, when its orbit has become a cycle of states (escape_orbit has the
-// reason).  A block in which no lane changes costs one branch beyond its steps and
+// set to max_iter, when its orbit has become a cycle of states.
+//
+// The cycle test: a block that ends inside compares its end state with a held earlier
+// one.  A step is a function of the state alone, so a state that comes back makes the
+// orbit a cycle whose states have all passed the bailout test or lie between block ends
+// that did (escape is permanent): it never escapes, and the loop's result is the one at
+// max_iter.  (The comparison takes -0 for 0; a zero's sign never changes a magnitude of
+// later states.)  Most interior orbits become such cycles long before max_iter: the
+// attracting cycle is reached to the last bit.
+//
+// A block in which no lane changes costs one branch beyond its steps and
 // three compares: while many waves run the loop is bound by VALU issue, but the few
 // waves left with the longest orbits set a launch's length, and a lone wave waits
 // for every scalar instruction.  Whole wave.
@@ -529,6 +433,30 @@ __device__ __forceinline__ bool finish_orbit(LaneOrbit<Real> &o, uint64_t failed
         checked_steps<Real, kFused>(o.x, o.y, o.cx, o.cy, o.i, max_iter, bsq, escaped, mag2);
     }
     return escaped;
+}
+
+// The reference loop  while (i < maxIter && x*x+y*y < R^2) { step; ++i; }  for every
+// active lane from its own state, with unchecked blocks of K steps when `blocks` holds
+// (escape is permanent for these inputs); max_iter and `blocks` are the same for all of
+// them (one tile per launch).
+template <class Real, int K, bool kFused>
+__device__ __forceinline__ Orbit<Real> escape_orbit(Real x, Real y, Real cx, Real cy,
+                                                     uint max_iter, Real bailout_sq,
+                                                     bool blocks) {
+    LaneOrbit<Real> o;
+    o.x = o.sx = o.mx = x;
+    o.y = o.sy = o.my = y;
+    o.cx = cx;
+    o.cy = cy;
+    o.i = 0;
+    o.template begin<K>(max_iter, kCycleFirst);
+    const uint64_t active = ballot(true);
+    uint64_t run = blocks && max_iter >= (uint)K ? active : 0ull, failed = 0, ended = active & ~run;
+    run_blocks<Real, K, kFused>(o, run, failed, ended, run, lanes(run), max_iter, bailout_sq);
+    Orbit<Real> r;
+    r.escaped = finish_orbit<Real, K, kFused>(o, failed, max_iter, bailout_sq, r.mag2);
+    r.n = o.i;
+    return r;
 }
 
 }  // namespace cu

@@ -220,7 +220,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // of the few waves with the longest orbits (a lone wave takes about 39 cycles per
 // step).  So which lanes run, failed or ended is kept in scalar masks, a block
 // without a change costs one branch beyond its steps, and an orbit that has become
-// a cycle of states stops there (escape_orbit has the reason).  1920x1080 default
+// a cycle of states stops there (run_blocks has the reason).  1920x1080 default
 // view, FP32, maxIter 1600, 5 adaptive spp: 408 -> 290 us (392 without the cycle
 // test); a bounded Julia set at 1280x720 308 -> 90 us; the 4096^2 frame's view in
 // 4K, FP64, 4 spp 1572 -> 1547 us, its 1080p zoom frames 450 -> 392 us.

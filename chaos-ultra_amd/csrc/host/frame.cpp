@@ -139,6 +139,7 @@ void enqueue_render(cu_frame f, const cu_frame_tune &tn, const uint32_t *d_palet
     cu_function combine = function(f->engine, "combinePending");
     uint32_t *counters = (uint32_t *)f->d_counters;
     const uint32_t n_tiles = (uint32_t)f->tiles.size();
+    const uint32_t cus = (uint32_t)std::max(1, compute_units());
 
     fill(f, stream, f->d_control, 0, kControlWords);
     if (events) check(hipEventRecord(f->ev_start, st), "hipEventRecord");
@@ -166,10 +167,11 @@ void enqueue_render(cu_frame f, const cu_frame_tune &tn, const uint32_t *d_palet
         void *q = f->d_queue[0];
         uint32_t *c = counters;
         void *params[] = {&a, &total_blocks, &q, &c};
-        launch(f->engine, pass1, dim3((total_blocks + 3) / 4), dim3(256), params, stream, false);
+        const uint32_t groups = (total_blocks + 3) / 4;
+        const uint32_t lds = few_blocks(dim3(groups)) ? lds_for(4) : groups <= 64 * cus ? lds_for(5) : 0;
+        launch(f->engine, pass1, dim3(groups), dim3(256), params, stream, false, lds);
     }
     if (events) check(hipEventRecord(f->ev_pass1, st), "hipEventRecord");
-    const uint32_t cus = (uint32_t)std::max(1, compute_units());
     // tail passes p = 1..tail_passes: pass p reads queue (p-1) & 1 with fill set
     // p-1 and writes queue p & 1 with fill set p.  Without a drain the last of
     // them runs every orbit to its end; with one, all hand off and the drain

@@ -16,7 +16,7 @@ namespace {
 // Device-side argument block of perturb{Float,Double} / deepDirectDouble*.
 struct DeepArgs {
     const void *orbit;
-    const uint32_t *orbit_len;
+    const void *info;
     uint32_t *counts;
     double *smooth;
     unsigned char *glitch;
@@ -73,7 +73,7 @@ struct cu_deep_s {
     bool fused = false;  // direct form: fused step variant
     size_t entry_bytes = 32;
     void *d_orbit[2] = {nullptr, nullptr};  // primary, secondary
-    void *d_len = nullptr;                  // u32[2]
+    void *d_len = nullptr;                  // two OrbitInfo
     void *d_counts = nullptr, *d_smooth = nullptr, *d_glitch = nullptr;
     void *d_iters = nullptr;                // CU_ITER_SLOTS u64
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -128,13 +128,16 @@ const char *orbit_kernel(const cu_deep_s *d) {
     return d->method == CU_DEEP_PERTURB_F32 ? "referenceOrbitFloat" : "referenceOrbitDouble";
 }
 
+// The OrbitInfo (4 words, the first the index of the last entry) of orbit `slot`.
+uint32_t *orbit_info(const cu_deep_s *d, int slot) { return (uint32_t *)d->d_len + 4 * slot; }
+
 void launch_orbit(cu_deep d, cu_stream s, int slot, double cx_hi, double cx_lo, double cy_hi,
                   double cy_lo, uint32_t mi) {
     cu_function f = function(d->engine, orbit_kernel(d));
     double bsq = d->desc.bailout_sq;
     void *orbit = d->d_orbit[slot];
-    uint32_t *len = (uint32_t *)d->d_len + slot;
-    void *params[] = {&cx_hi, &cx_lo, &cy_hi, &cy_lo, &mi, &bsq, &orbit, &len};
+    void *info = orbit_info(d, slot);
+    void *params[] = {&cx_hi, &cx_lo, &cy_hi, &cy_lo, &mi, &bsq, &orbit, &info};
     launch(d->engine, f, dim3(1), dim3(64), params, s, false);
 }
 
@@ -142,7 +145,7 @@ DeepArgs base_args(cu_deep d, const uint32_t *pal, uint32_t plen, uint32_t *rgba
     const cu_deep_desc &c = d->desc;
     DeepArgs a{};
     a.orbit = d->d_orbit[0];
-    a.orbit_len = (const uint32_t *)d->d_len;
+    a.info = orbit_info(d, 0);
     a.counts = (uint32_t *)d->d_counts;
     a.smooth = (double *)d->d_smooth;
     a.glitch = (unsigned char *)d->d_glitch;
@@ -247,7 +250,7 @@ int cu_deep_create(cu_engine e, const cu_deep_desc *desc, int method, cu_deep *o
             if (!(desc->flags & CU_DEEP_REBASE) && desc->max_references > 0)
                 d->d_orbit[1] = device_alloc(entries * d->entry_bytes);
         }
-        d->d_len = device_alloc(2 * sizeof(uint32_t));
+        d->d_len = device_alloc(2 * 4 * sizeof(uint32_t));
         d->d_counts = device_alloc(pixels * 4);
         d->d_smooth = device_alloc(pixels * 8);
         d->d_glitch = device_alloc(pixels);
@@ -306,9 +309,9 @@ int cu_deep_render(cu_deep d, const uint32_t *d_palette, uint32_t palette_length
                           c.max_iter <= d->orbit_mi;
         fill_u32(d->engine, stream, d->d_iters, 0, CU_ITER_SLOTS * 2);
         if (keep)
-            fill_u32(d->engine, stream, (uint32_t *)d->d_len + 1, 0, 1);
+            fill_u32(d->engine, stream, orbit_info(d, 1), 0, 4);
         else
-            fill_u32(d->engine, stream, d->d_len, 0, 2);
+            fill_u32(d->engine, stream, d->d_len, 0, 8);
         check(hipEventRecord(d->ev[0], st), "hipEventRecord");
         d->references = 0;
         d->glitched = 0;
@@ -345,7 +348,7 @@ int cu_deep_render(cu_deep d, const uint32_t *d_palette, uint32_t palette_length
                 ++d->references;
                 DeepArgs g = a;
                 g.orbit = d->d_orbit[1];
-                g.orbit_len = (const uint32_t *)d->d_len + 1;
+                g.info = orbit_info(d, 1);
                 g.ref_ox = ox;
                 g.ref_oy = oy;
                 g.only_glitched = 1;
@@ -377,9 +380,9 @@ int cu_deep_stats(cu_deep d, cu_deep_report *out) {
         cu_deep_report s{};
         if (cu_iters_total((const unsigned long long *)d->d_iters, &s.iterations) != CU_OK)
             fail(CU_ERR_DEVICE, cu_last_error());
-        uint32_t len[2] = {0, 0};
-        check(hipMemcpy(len, d->d_len, sizeof(len), hipMemcpyDeviceToHost), "hipMemcpy D2H");
-        s.reference_length = len[0];
+        uint32_t len = 0;
+        check(hipMemcpy(&len, d->d_len, sizeof(len), hipMemcpyDeviceToHost), "hipMemcpy D2H");
+        s.reference_length = len;
         s.references = d->references;
         s.glitched = d->glitched;
         check(hipEventElapsedTime(&s.orbit_ms, d->ev[0], d->ev[1]), "hipEventElapsedTime");

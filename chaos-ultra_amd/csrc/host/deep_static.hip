@@ -31,7 +31,7 @@
 
 namespace {
 
-// The orbit at its widest (FP64 entries, 32 B), then M in its own 256-byte line.
+// The orbit at its widest (FP64 entries, 32 B), then its OrbitInfo in its own 256-byte line.
 constexpr size_t kOrbitBytes = ((size_t)CU_DEEP_STATIC_MAX_ITER + 1) * sizeof(OrbitEntry<double>);
 constexpr size_t kScratchBytes = kOrbitBytes + 256;
 static_assert(kScratchBytes == CU_DEEP_STATIC_BYTES, "scratch size in the header");
@@ -62,8 +62,8 @@ template <class Real>
 __global__ __launch_bounds__(64) void staticReferenceOrbit(double cx_hi, double cx_lo,
                                                            double cy_hi, double cy_lo,
                                                            uint max_iter, double bailout_sq,
-                                                           OrbitEntry<Real> *orbit, uint *length) {
-    reference_orbit<Real>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit, length);
+                                                           OrbitEntry<Real> *orbit, OrbitInfo *info) {
+    reference_orbit<Real>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit, info);
 }
 
 // The block shapes and LDS stages of perturbFloat / perturbDouble (perturb.hip).
@@ -81,14 +81,14 @@ void render(const cu_deep_desc &c, unsigned char *base, uint32_t *counts, double
             const uint32_t *palette, uint32_t palette_length, uint32_t *rgba,
             unsigned long long *iters, hipStream_t st) {
     OrbitEntry<Real> *orbit = (OrbitEntry<Real> *)base;
-    uint *len = (uint *)(base + kOrbitBytes);
+    OrbitInfo *info = (OrbitInfo *)(base + kOrbitBytes);
     hipLaunchKernelGGL(staticReferenceOrbit<Real>, dim3(1), dim3(64), 0, st, c.centre_x,
                        c.centre_x_lo, c.centre_y, c.centre_y_lo, c.max_iter, c.bailout_sq, orbit,
-                       len);
+                       info);
     cu::check(hipGetLastError(), "launch staticReferenceOrbit");
     DeepArgs a{};
     a.orbit = orbit;
-    a.orbit_len = len;
+    a.info = info;
     a.counts = counts;
     a.smooth = smooth;
     a.glitch = nullptr;

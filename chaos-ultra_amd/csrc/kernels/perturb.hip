@@ -1,7 +1,7 @@
 // perturb.hip — entry points of the deep-zoom render form (part of
 // escape_family.hsaco); the device code is in perturb_core.hpp.
 //
-//   referenceOrbit{Float,Double}   one lane: double-double orbit of C -> entries, M
+//   referenceOrbit{Float,Double}   one wave: double-double orbit of C -> entries, M and its cycle
 //   perturb{Float,Double}          lane per pixel (8x8 pixels per wave, 16x16 / 32x16 per block,
 //                                  orbit staged in LDS)
 //   deepDirectDouble               direct FP64 at the same pixel -> c mapping
@@ -9,13 +9,13 @@
 
 extern "C" __global__ __launch_bounds__(64) void referenceOrbitFloat(
     double cx_hi, double cx_lo, double cy_hi, double cy_lo, uint max_iter, double bailout_sq,
-    OrbitEntry<float> *orbit, uint *length) {
-    reference_orbit<float>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit, length);
+    OrbitEntry<float> *orbit, OrbitInfo *info) {
+    reference_orbit<float>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit, info);
 }
 extern "C" __global__ __launch_bounds__(64) void referenceOrbitDouble(
     double cx_hi, double cx_lo, double cy_hi, double cy_lo, uint max_iter, double bailout_sq,
-    OrbitEntry<double> *orbit, uint *length) {
-    reference_orbit<double>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit, length);
+    OrbitEntry<double> *orbit, OrbitInfo *info) {
+    reference_orbit<double>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit, info);
 }
 // `orbit` repeats a.orbit as its own read-only argument, so uniform loads from
 // it can go through the scalar cache.  The second bound (8 waves per SIMD)

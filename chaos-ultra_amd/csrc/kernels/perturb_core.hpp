@@ -137,10 +137,8 @@ struct OrbitView {
 constexpr uint kOrbitRun = 8;
 
 template <class Real>
-__device__ void reference_orbit(double cx_hi, double cx_lo, double cy_hi, double cy_lo,
-                                uint max_iter, double bailout_sq, OrbitEntry<Real> *orbit,
-                                uint *length) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
+__device__ uint orbit_entries(double cx_hi, double cx_lo, double cy_hi, double cy_lo,
+                              uint max_iter, double bailout_sq, OrbitEntry<Real> *orbit) {
     const DD cx{cx_hi, cx_lo}, cy{cy_hi, cy_lo};
     DD x{0.0, 0.0}, y{0.0, 0.0};
     uint n = 0;
@@ -175,12 +173,78 @@ __device__ void reference_orbit(double cx_hi, double cx_lo, double cy_hi, double
         dd_orbit_step(x, y, cx, cy);
         ++n;
     }
-    *length = n;
+    return n;
+}
+
+// The reference orbit as the pixel kernels need it beside its entries: the index of the
+// last one, and the cycle it ends in: entries m and m + period are the same for all m
+// from `start` on (as far as entries go; period 0: no cycle was found, or the orbit
+// escapes).
+struct OrbitInfo {
+    uint last, period, start, pad;
+};
+
+// A point inside the set settles into a cycle, and rounded to the delta type its entries
+// repeat exactly long before the double-double values do.  One wave looks back from the
+// last entry for an equal one, at most kPeriodMax before it, then for the first pair a
+// period apart that differs.  For 50001 entries about 0.1 ms, where the orbit took 5 ms.
+constexpr uint kPeriodMax = 4096;
+
+template <class Real>
+__device__ void orbit_cycle(const OrbitEntry<Real> *orbit, uint M, uint &period, uint &start) {
+    const uint lane = threadIdx.x;
+    auto alike = [&](uint a, uint b) {
+        const OrbitEntry<Real> e = orbit[a], f = orbit[b];
+        return e.x == f.x && e.y == f.y && e.h == f.h;
+    };
+    period = start = 0;
+    const uint longest = min(M, kPeriodMax);
+    for (uint d = 1; d <= longest; d += 64) {
+        const uint64_t hit = cu::ballot(d + lane <= longest && alike(M - min(d + lane, M), M));
+        if (hit != 0) {
+            period = d + (uint)__builtin_ctzll(hit);
+            break;
+        }
+    }
+    if (period == 0) return;
+    constexpr uint kAhead = 4;  // wave-widths of entries looked at together
+    for (uint top = M - period + 1; top != 0;) {  // indices from `top` on have been found alike
+        uint64_t differ[kAhead];
+#pragma unroll
+        for (uint j = 0; j < kAhead; ++j) {
+            const uint back = j * 64 + lane + 1;
+            const uint m = top - min(back, top);
+            differ[j] = cu::ballot(back <= top && !alike(m, m + period));
+        }
+#pragma unroll
+        for (uint j = 0; j < kAhead; ++j)
+            if (differ[j] != 0) {
+                start = top - j * 64 - (uint)__builtin_ctzll(differ[j]);
+                return;
+            }
+        top -= min(top, kAhead * 64);
+    }
+}
+
+// One wave: its first lane computes the orbit, all look for the cycle.
+template <class Real>
+__device__ void reference_orbit(double cx_hi, double cx_lo, double cy_hi, double cy_lo,
+                                uint max_iter, double bailout_sq, OrbitEntry<Real> *orbit,
+                                OrbitInfo *info) {
+    if (blockIdx.x != 0) return;
+    uint n = 0;
+    if (threadIdx.x == 0)
+        n = orbit_entries<Real>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit);
+    __syncthreads();
+    const uint M = __builtin_amdgcn_readfirstlane(n);
+    uint period = 0, start = 0;
+    if (M == max_iter && M != 0) orbit_cycle<Real>(orbit, M, period, start);
+    if (threadIdx.x == 0) *info = {M, period, start, 0};
 }
 
 struct DeepArgs {
     const void *orbit;         // OrbitEntry<Real>[M + 1]
-    const uint *orbit_len;     // M
+    const OrbitInfo *info;
     uint *counts;              // W x H, row-major
     double *smooth;
     unsigned char *glitch;     // 1 = glitched (Pauldelbrot) in the last pass over the pixel
@@ -282,23 +346,32 @@ __device__ __forceinline__ int checked_step(const OrbitView<Real> &Z, uint M, Re
     return 0;
 }
 
-// K unchecked steps from orbit entry zp[0]; returns the ballot of lanes whose
-// rebase test fired at any of the K states.  No branches: the orbit loads of the
-// whole block can be issued ahead of the arithmetic.
-template <class Real, int K, class Ptr>
-__device__ __forceinline__ uint64_t unchecked_block(Ptr zp, Real &dx, Real &dy, Real dcx,
-                                                    Real dcy) {
+// K unchecked steps from orbit entry zp[0], the same for all lanes; returns the ballot of
+// lanes whose rebase test fired at any of the K states.  No branches: the orbit loads of
+// the whole block can be issued ahead of the arithmetic.  Entries are read 64 bytes at a
+// time, one scalar load for two FP64 or four FP32 ones: in 1e-10 and 1e-20 frames with
+// FP64 deltas 3 % less time than with two loads an entry, 1 to 3 % at 1e-6 (the other
+// waves cover the loads' latency; asking one group ahead was slower by a tenth).
+template <class Real, int K>
+__device__ __forceinline__ uint64_t unchecked_block(global_ptr<OrbitEntry<Real>> zp, Real &dx,
+                                                    Real &dy, Real dcx, Real dcy) {
+    constexpr int kTogether = 64 / (int)sizeof(OrbitEntry<Real>);
+    typedef Real Entries __attribute__((ext_vector_type(4 * kTogether), aligned(4 * sizeof(Real))));
     uint64_t flagged = 0;
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const OrbitEntry<Real> e = load_entry<Real>(zp + k);
-        flagged |= cu::ballot(rebase_test(e.x, e.y, e.h, dx, dy));
-        const Real ax = cu::fma_r((Real)2, e.x, dx);
-        const Real ay = cu::fma_r((Real)2, e.y, dy);
-        const Real ndx = cu::fma_r(ax, dx, cu::fma_r(-ay, dy, dcx));
-        const Real ndy = cu::fma_r(ax, dy, cu::fma_r(ay, dx, dcy));
-        dx = ndx;
-        dy = ndy;
+    for (int k = 0; k < K; k += kTogether) {
+        const Entries z = *(global_ptr<Entries>)(zp + k);
+#pragma unroll
+        for (int j = 0; j < kTogether; ++j) {
+            const Real x = z[4 * j], y = z[4 * j + 1], h = z[4 * j + 2];
+            flagged |= cu::ballot(rebase_test(x, y, h, dx, dy));
+            const Real ax = cu::fma_r((Real)2, x, dx);
+            const Real ay = cu::fma_r((Real)2, y, dy);
+            const Real ndx = cu::fma_r(ax, dx, cu::fma_r(-ay, dy, dcx));
+            const Real ndy = cu::fma_r(ax, dy, cu::fma_r(ay, dx, dcy));
+            dx = ndx;
+            dy = ndy;
+        }
     }
     return flagged;
 }
@@ -365,18 +438,29 @@ __device__ __forceinline__ uint64_t rebasing_block(Ptr orbit, uint M, const Orbi
 // body; the last max_iter % K steps are checked ones too.  A lane whose rebase delta
 // has come back is at a cycle's end (HeldDelta).
 //
+// A lane that does not rebase, with the reference inside the set, is the other kind of
+// cycle: along the reference's own cycle its future is a function of its delta and its
+// place in the cycle.  Lanes that are on it when a delta is to be held hold their present
+// one (`along`), and it is looked for again a whole number of periods later, at the block
+// ends `stride` apart.  (A pixel's index is never above its iteration count, so with a
+// reference that runs to max_iter the end of the entries is not reached before the last
+// iteration, and entries a period apart are the same entry to it.)
+//
 // Without rebasing every step is a checked one (the glitch test needs each).
 //
-// Bound by VALU issue; 1920x1080, without the reference orbit's time, FP32 / FP64
-// deltas: 1e-10 (each pixel rebases on its own) 1.50 / 2.24 -> 1.09 / 1.92 ms, a
-// shallow frame of width 1 2.85 / 3.80 -> 0.70 / 1.15 ms, 1e-20 (few rebases) 1.20 / 2.03
-// -> 1.16 / 1.94 ms; before, a block stopped for the whole wave at its first rebase,
-// and each escape was replayed as it came, 32 checked steps for one lane.  1e-6, three
-// quarters interior, 18.7 / 32.7 -> 8.9 / 19.3 ms, 11.0 / 22.0 of it by the cycle test.
+// Bound by VALU issue, and by the longest waves once the others have ended; 1920x1080,
+// without the reference orbit's time, FP32 / FP64 deltas: 1e-10 (each pixel rebases on
+// its own) 1.50 / 2.24 -> 1.07 / 1.83 ms, a shallow frame of width 1 2.85 / 3.80 ->
+// 0.43 / 0.71 ms (0.70 / 1.15 without the cycles along the reference's), 1e-20 (few
+// rebases) 1.20 / 2.03 -> 1.15 / 1.87 ms; before, a block stopped for the whole wave at
+// its first rebase, and each escape was replayed as it came, 32 checked steps for one
+// lane.  1e-6, three quarters interior, 18.7 / 32.7 -> 8.8 / 19.1 ms, 11.0 / 22.0 of it
+// by the cycle test.
 template <class Real, int K>
-__device__ int perturb_pixel(const OrbitView<Real> &Z, uint M, Real dcx, Real dcy, uint max_iter,
-                             Real bsq, bool rebase, Real geps, bool active, uint &n_out,
+__device__ int perturb_pixel(const OrbitView<Real> &Z, const OrbitInfo &info, Real dcx,
+                             Real dcy, uint max_iter, Real bsq, bool rebase, Real geps, bool active, uint &n_out,
                              Real &mag_out) {
+    const uint M = info.last;
     Real dx = 0, dy = 0;
     uint m = 0, n_lane = 0;
     int state = active ? 0 : 4;
@@ -389,6 +473,10 @@ __device__ int perturb_pixel(const OrbitView<Real> &Z, uint M, Real dcx, Real dc
         Real rx = 0, ry = 0;             // delta of the lane's last rebase
         HeldDelta<Real> held;
         uint hold = 0;                   // iteration count from which the next one is held
+        uint64_t along = 0;              // lanes that hold their delta on the reference's cycle
+        uint due = 0;                    // iteration count at which theirs is looked for
+        const uint stride = info.period * ((uint)K >> min((uint)__builtin_ctz(info.period | (uint)K),
+                                                          (uint)__builtin_ctz((uint)K)));
         uint streak = 0;                 // consecutive blocks rerun for a rebase
         const OrbitEntry<Real> z1 = load_entry<Real>(Z.global + min(1u, M));
         while (run != 0 && max_iter - n >= (uint)K) {
@@ -443,16 +531,33 @@ __device__ int perturb_pixel(const OrbitView<Real> &Z, uint M, Real dcx, Real dc
             rebased &= run;
             if (rebased != 0) {
                 cu::seldom();
-                const uint64_t cycle = rebased & cu::ballot(held.is(rx, ry));
+                const uint64_t cycle = rebased & ~along & cu::ballot(held.is(rx, ry));
                 if (cu::in_mask(cycle)) {
                     n_lane = max_iter;
                     state = 2;
                 }
                 run &= ~cycle;
+                if (cu::in_mask(along & rebased)) held.take(rx, ry);
+                along &= ~rebased;
+            }
+            if (n == due) {
+                cu::seldom();
+                const uint64_t cycle = run & along & cu::ballot(held.is(dx, dy));
+                if (cu::in_mask(cycle)) {
+                    n_lane = max_iter;
+                    state = 2;
+                }
+                run &= ~cycle;
+                due += stride;
             }
             if (n >= hold) {
                 cu::seldom();
-                held.take(rx, ry);
+                along = info.period != 0 ? run & cu::ballot(m >= info.start) : 0;
+                if (cu::in_mask(along))
+                    held.take(dx, dy);
+                else
+                    held.take(rx, ry);
+                due = n + stride;
                 hold = n + n / 2;
             }
         }
@@ -500,8 +605,8 @@ __device__ __forceinline__ void deep_pixel_coords(uint &px, uint &py) {
 template <class Real, int K, uint WX, uint WY, uint LdsBytes>
 __device__ void perturb_frame(const DeepArgs a, const OrbitEntry<Real> *__restrict__ orbit) {
     __shared__ OrbitEntry<Real> lds[LdsBytes / sizeof(OrbitEntry<Real>)];
-    const uint M = *a.orbit_len;
-    const uint staged = min(M + 1u, LdsBytes / (uint)sizeof(OrbitEntry<Real>));
+    const OrbitInfo info = *a.info;
+    const uint staged = min(info.last + 1u, LdsBytes / (uint)sizeof(OrbitEntry<Real>));
     for (uint k = threadIdx.x; k < staged; k += blockDim.x) lds[k] = orbit[k];
     __syncthreads();
     const OrbitView<Real> view{(global_ptr<OrbitEntry<Real>>)orbit,
@@ -521,7 +626,7 @@ __device__ void perturb_frame(const DeepArgs a, const OrbitEntry<Real> *__restri
     uint n = 0;
     Real mag = 0;
     const int state = perturb_pixel<Real, K>(
-        view, M, dcx, dcy, a.max_iter, (Real)a.bailout_sq,
+        view, info, dcx, dcy, a.max_iter, (Real)a.bailout_sq,
         (a.flags & kDeepRebase) != 0, (Real)a.glitch_eps, active, n, mag);
     if (active) deep_write(a, o, state, n, (double)mag);
     cu::add_iterations(a.iters, active ? (uint64_t)n : 0u);

@@ -171,3 +171,31 @@ def test_frame_pipeline(gpu, engine, oracle, tune, spp, precision):
 def test_perturbation(gpu, engine, oracle, centre, width, limit, method):
     """Rebased deltas that come back end the pixel with the checked loop's result."""
     deep_case(gpu, engine, oracle, gpu.make_deep(*centre, width, 45, 27, limit, 256.0), method)
+
+
+# references that settle into cycles of 1, 2, 3, 4, 10 and 78 entries, at different rates; the
+# limits are no multiples of a block's 32 steps, and the second frame keeps the first's orbit
+@pytest.mark.parametrize("centre,width", [
+    ((-0.4, 0.05), 0.9), ((-1.02, 0.03), 0.3), ((-0.123, 0.745), 0.12),
+    ((0.2823, 0.5301), 0.05), ((-0.5355, 0.6085), 0.02), ((-0.7436440753, 0.1318253789), 1e-6)])
+@pytest.mark.parametrize("method", [32, 64])
+def test_perturbation_along_a_periodic_reference(gpu, engine, oracle, centre, width, method):
+    """A delta that comes back a whole number of the reference's periods later ends the pixel
+    with the checked loop's result, also with an orbit longer than the frame's limit."""
+    om = oracle.DEEP_PERTURB_F32 if method == 32 else oracle.DEEP_PERTURB_F64
+    desc = gpu.make_deep(*centre, width, 45, 27, 9001, 256.0)
+    desc.flags |= gpu.abi.DEEP_REUSE_ORBIT
+    frame = gpu.DeepFrame(engine, desc, method)
+    ys, xs = np.mgrid[0:desc.height, 0:desc.width]
+    for limit in (9001, 2999):
+        desc.max_iter = limit
+        frame.retarget(desc)
+        frame.render()
+        report = frame.report()
+        assert report.references == (1 if limit == 9001 else 0)
+        orbit = frame.orbit() if limit == 9001 else orbit
+        wc, _, _, wit = oracle.deep_pixels(om, xs.ravel(), ys.ravel(), desc, orbit,
+                                           report.reference_length)
+        assert np.array_equal(frame.counts().ravel(), wc)
+        assert report.iterations == wit
+    frame.close()

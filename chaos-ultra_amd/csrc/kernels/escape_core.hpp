@@ -366,53 +366,102 @@ struct LaneOrbit {
 // later states.)  Most interior orbits become such cycles long before max_iter: the
 // attracting cycle is reached to the last bit.
 //
+// A block's start is kept for the lanes that fail in it.  kTurns: blocks go from (x, y)
+// to (sx, sy) and back in turn, so keeping it takes no copies (4 of about 105 VALU
+// instructions a block); lanes that end with their state in (sx, sy) are turned round
+// at the end.  For callers whose lanes run to their end here: FP64 / FP32 frames 1.8 / 2.9 %
+// faster (4096^2 at 4 spp 2851 -> 2801 us, 1501x1103 at 2 spp 518 -> 503 us), direct deep
+// frames 3.7 % (8.8 -> 8.5 ms), a 1024^2 tile 2 %.  Callers that come back to refill lanes
+// copy: turning round at each return cost a zoom's frames 1 %, and batches gained nothing.
+//
 // A block in which no lane changes costs one branch beyond its steps and
 // three compares: while many waves run the loop is bound by VALU issue, but the few
 // waves left with the longest orbits set a launch's length, and a lone wave waits
 // for every scalar instruction.  Whole wave.
-template <class Real, int K, bool kFused>
+template <class Real, int K, bool kFused, bool kTurns>
 __device__ __forceinline__ void run_blocks(LaneOrbit<Real> &o, uint64_t &run, uint64_t &failed,
                                            uint64_t &ended, uint64_t counted, uint enough,
                                            uint max_iter, Real bsq) {
     Real x2 = o.x * o.x, y2 = o.y * o.y;  // squares of the current state, carried
     enough = min(enough, lanes(counted));  // with no lane running, all counted ones wait
     if (lanes(counted & ~run) >= enough) return;
-    for (;;) {
-        uint64_t inside, due, again;
-        do {
-            if (in_mask(run)) {
-                o.sx = o.x;
-                o.sy = o.y;
+    uint64_t turned = 0;  // lanes that ended with their state in (sx, sy)
+    uint64_t inside, due, again;
+    auto block = [&](const Real &fx, const Real &fy, Real &tx, Real &ty) {
+        if (in_mask(run)) {
+            Real x = fx, y = fy;
 #pragma unroll
-                for (int k = 0; k < K / 2; ++k)
-                    quad_step_sq<Real, kFused>(o.x, o.y, x2, y2, o.cx, o.cy);
-                o.mx = o.x;
-                o.my = o.y;
+            for (int k = 0; k < K / 2; ++k) quad_step_sq<Real, kFused>(x, y, x2, y2, o.cx, o.cy);
+            o.mx = x;
+            o.my = y;
 #pragma unroll
-                for (int k = K / 2; k < K; ++k)
-                    quad_step_sq<Real, kFused>(o.x, o.y, x2, y2, o.cx, o.cy);
-                o.i += K;
-            }
-            inside = ballot(x2 + y2 < bsq);
-            due = ballot(o.i >= o.until);
-            again = ballot(o.y == o.hy);
-        } while ((run & (~inside | due | again)) == 0);
+            for (int k = K / 2; k < K; ++k) quad_step_sq<Real, kFused>(x, y, x2, y2, o.cx, o.cy);
+            tx = x;
+            ty = y;
+            o.i += K;
+        }
+        inside = ballot(x2 + y2 < bsq);
+        due = ballot(o.i >= o.until);
+        again = ballot(ty == o.hy);
+        return (run & (~inside | due | again)) != 0;
+    };
+    auto leave = [&](const Real &x, const Real &y) {  // lanes whose state changes at a block's end
         failed |= run & ~inside;
         run &= inside;
         if ((run & (due | again)) != 0) {
             seldom();
-            const uint64_t cycle = run & again & ballot(o.x == o.hx);
+            const uint64_t cycle = run & again & ballot(x == o.hx);
             if (in_mask(cycle)) o.i = max_iter;  // the loop's result: max_iter steps, no escape
             const uint64_t spent = run & ballot(o.i > max_iter - (uint)K);
             ended |= spent;
             run &= ~spent;
             if (in_mask(run & due)) {
-                o.hx = o.x;
-                o.hy = o.y;
+                o.hx = x;
+                o.hy = y;
                 o.until = min(next_hold<K>(o.i), max_iter - (uint)K + 1u);
             }
         }
-        if (lanes(counted & ~run) >= enough) return;
+        return lanes(counted & ~run) >= enough;
+    };
+    if constexpr (kTurns) {
+        for (;;) {
+            if (block(o.x, o.y, o.sx, o.sy)) {
+                const uint64_t before = run;
+                const bool done = leave(o.sx, o.sy);
+                turned |= done ? before : before & ~run;
+                if (done) break;
+            }
+            if (block(o.sx, o.sy, o.x, o.y) && leave(o.x, o.y)) break;
+        }
+        if (in_mask(turned)) {
+            const Real x = o.x, y = o.y;
+            o.x = o.sx;
+            o.y = o.sy;
+            o.sx = x;
+            o.sy = y;
+        }
+    } else {
+        for (;;) {
+            do {
+                if (in_mask(run)) {
+                    o.sx = o.x;
+                    o.sy = o.y;
+#pragma unroll
+                    for (int k = 0; k < K / 2; ++k)
+                        quad_step_sq<Real, kFused>(o.x, o.y, x2, y2, o.cx, o.cy);
+                    o.mx = o.x;
+                    o.my = o.y;
+#pragma unroll
+                    for (int k = K / 2; k < K; ++k)
+                        quad_step_sq<Real, kFused>(o.x, o.y, x2, y2, o.cx, o.cy);
+                    o.i += K;
+                }
+                inside = ballot(x2 + y2 < bsq);
+                due = ballot(o.i >= o.until);
+                again = ballot(o.y == o.hy);
+            } while ((run & (~inside | due | again)) == 0);
+            if (leave(o.x, o.y)) return;
+        }
     }
 }
 
@@ -452,7 +501,7 @@ __device__ __forceinline__ Orbit<Real> escape_orbit(Real x, Real y, Real cx, Rea
     o.template begin<K>(max_iter, kCycleFirst);
     const uint64_t active = ballot(true);
     uint64_t run = blocks && max_iter >= (uint)K ? active : 0ull, failed = 0, ended = active & ~run;
-    run_blocks<Real, K, kFused>(o, run, failed, ended, run, lanes(run), max_iter, bailout_sq);
+    run_blocks<Real, K, kFused, true>(o, run, failed, ended, run, lanes(run), max_iter, bailout_sq);
     Orbit<Real> r;
     r.escaped = finish_orbit<Real, K, kFused>(o, failed, max_iter, bailout_sq, r.mag2);
     r.n = o.i;

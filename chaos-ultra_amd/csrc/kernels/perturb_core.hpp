@@ -458,8 +458,8 @@ __device__ __forceinline__ uint64_t rebasing_block(Ptr orbit, uint M, const Orbi
 // by the cycle test.
 template <class Real, int K>
 __device__ int perturb_pixel(const OrbitView<Real> &Z, const OrbitInfo &info, Real dcx,
-                             Real dcy, uint max_iter, Real bsq, bool rebase, Real geps, bool active, uint &n_out,
-                             Real &mag_out) {
+                             Real dcy, uint max_iter, Real bsq, bool rebase, Real geps,
+                             bool active, uint &n_out, Real &mag_out) {
     const uint M = info.last;
     Real dx = 0, dy = 0;
     uint m = 0, n_lane = 0;
@@ -475,8 +475,7 @@ __device__ int perturb_pixel(const OrbitView<Real> &Z, const OrbitInfo &info, Re
         uint hold = 0;                   // iteration count from which the next one is held
         uint64_t along = 0;              // lanes that hold their delta on the reference's cycle
         uint due = 0;                    // iteration count at which theirs is looked for
-        const uint stride = info.period * ((uint)K >> min((uint)__builtin_ctz(info.period | (uint)K),
-                                                          (uint)__builtin_ctz((uint)K)));
+        const uint stride = info.period * ((uint)K >> __builtin_ctz(info.period | (uint)K));
         uint streak = 0;                 // consecutive blocks rerun for a rebase
         const OrbitEntry<Real> z1 = load_entry<Real>(Z.global + min(1u, M));
         while (run != 0 && max_iter - n >= (uint)K) {

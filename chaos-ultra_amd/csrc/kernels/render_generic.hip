@@ -369,7 +369,7 @@ __device__ uint sample_the_fractal(WaveLds &lds, int site, Point<uint> grid, Rec
         }
 
         // ---- unchecked blocks until kRefill lanes wait (idle ones count while work is left) ----
-        cu::run_blocks<Real, K, kFused>(o, run, failed, ended, more ? ~0ull : run | ended, kRefill,
+        cu::run_blocks<Real, K, kFused, false>(o, run, failed, ended, more ? ~0ull : run | ended, kRefill,
                                         max_iter, bsq);
 
         // ---- finish the pending orbits and post their iteration counts ----

@@ -25,6 +25,7 @@
 
 #include "common.hpp"
 #include "handles.hpp"
+#include "render_form.hpp"
 
 namespace cu {
 namespace {
@@ -114,13 +115,13 @@ const char *const kKernelNames[] = {"fractalRenderMainFloat",     "fractalRender
                                     "fractalRenderAdvancedFloat", "fractalRenderAdvancedDouble",
                                     "fractalRenderUnderSampled",  "compose",
                                     "debug"};
-// The same four render kernels for 32 x 4-thread blocks (this build's modules
+// The same four render kernels in the forms of render_form.hpp (this build's modules
 // export them; a module without them renders through the kernels above).
-const char *const kStripKernelNames[] = {"fractalRenderMainFloatStrip",
-                                         "fractalRenderMainDoubleStrip",
-                                         "fractalRenderAdvancedFloatStrip",
-                                         "fractalRenderAdvancedDoubleStrip"};
-constexpr int kStripRows = 4;  // rows of a strip block
+const char *const kFormKernelNames[] = {
+    "fractalRenderMainFloatStrip",     "fractalRenderMainDoubleStrip",
+    "fractalRenderAdvancedFloatStrip", "fractalRenderAdvancedDoubleStrip",
+    "fractalRenderMainFloatGroup",     "fractalRenderMainDoubleGroup",
+    "fractalRenderAdvancedFloatGroup", "fractalRenderAdvancedDoubleGroup"};
 
 class Module {
   public:
@@ -148,7 +149,7 @@ class Module {
             }
             kernels_[k] = f;
         }
-        for (const char *k : kStripKernelNames) {
+        for (const char *k : kFormKernelNames) {
             cu_function f = nullptr;
             if (cu_module_get_function(module_, k, &f) == CU_OK) kernels_[k] = f;
         }
@@ -342,7 +343,8 @@ struct RectT {
 
 struct RenderKernel {
     cu_function fn = nullptr;
-    cu_function strip = nullptr;  // the same kernel for 32 x 4-thread blocks, if the module has it
+    cu_function strip = nullptr;  // its other forms (render_form.hpp), if the module has them
+    cu_function group = nullptr;
     bool is_float = false;
     bool advanced = false;
     int width = 0, height = 0;
@@ -395,9 +397,9 @@ struct RenderKernel {
         }
     }
 
-    // Launch and synchronise: the strip kernel over ceil(W/32) x ceil(H/4) blocks
-    // of 32 x 4 threads when the module has it (the same pixels, vote groups and
-    // results), else the reference's geometry.
+    // Launch and synchronise: one of the forms over ceil(W/32) x ceil(H/4) blocks when
+    // the module has it (the same pixels, vote groups and results), else the
+    // reference's geometry.
     void launch() {
         PointT<uint32_t> size{(uint32_t)width, (uint32_t)height};
         RectT<double> rd{seg.lbx, seg.lby, seg.rtx, seg.rty};
@@ -412,8 +414,14 @@ struct RenderKernel {
         unsigned gx = (unsigned)((width + kBlockDim - 1) / kBlockDim);
         unsigned gy = (unsigned)((height + kBlockDim - 1) / kBlockDim);
         const int64_t strip_rows = ((int64_t)height + kStripRows - 1) / kStripRows;
+        const bool reuse = advanced && (flags & CU_FLAG_SAMPLE_REUSE) != 0;
         int rc;
-        if (strip && strip_rows <= kMaxGridDim)
+        if (group && strip_rows <= kMaxGridDim &&
+            one_group_waves(width, height, max_ss, reuse, {seg.lbx, seg.lby, seg.rtx, seg.rty},
+                            {origin.lbx, origin.lby, origin.rtx, origin.rty}))
+            rc = cu_launch_kernel(group, gx, (unsigned)strip_rows, 1, kBlockDim, kGroupTRows, 1, 0,
+                                  params);
+        else if (strip && strip_rows <= kMaxGridDim)
             rc = cu_launch_kernel(strip, gx, (unsigned)strip_rows, 1, kBlockDim, kStripRows, 1, 0,
                                   params);
         else
@@ -449,15 +457,19 @@ class Renderer {
     explicit Renderer(Module *module) : module_(module) {
         main_f_.fn = module->kernel("fractalRenderMainFloat");
         main_f_.strip = module->kernel_if("fractalRenderMainFloatStrip");
+        main_f_.group = module->kernel_if("fractalRenderMainFloatGroup");
         main_f_.is_float = true;
         main_d_.fn = module->kernel("fractalRenderMainDouble");
         main_d_.strip = module->kernel_if("fractalRenderMainDoubleStrip");
+        main_d_.group = module->kernel_if("fractalRenderMainDoubleGroup");
         adv_f_.fn = module->kernel("fractalRenderAdvancedFloat");
         adv_f_.strip = module->kernel_if("fractalRenderAdvancedFloatStrip");
+        adv_f_.group = module->kernel_if("fractalRenderAdvancedFloatGroup");
         adv_f_.is_float = true;
         adv_f_.advanced = true;
         adv_d_.fn = module->kernel("fractalRenderAdvancedDouble");
         adv_d_.strip = module->kernel_if("fractalRenderAdvancedDoubleStrip");
+        adv_d_.group = module->kernel_if("fractalRenderAdvancedDoubleGroup");
         adv_d_.advanced = true;
         compose_ = module->kernel("compose");
         debug_ = module->kernel("debug");

@@ -42,6 +42,7 @@
 #include "common.hpp"
 #include "engine_helpers.hpp"
 #include "handles.hpp"
+#include "render_form.hpp"
 
 namespace {
 
@@ -52,7 +53,6 @@ constexpr int kBlockDim = 32;  // reference launch geometry (CudaFractalRenderer
 // which the other sessions' renders leave late: beside them compose took 207 us a frame
 // on average, 5 us alone.
 constexpr int kComposeRows = 8;
-constexpr int kStripRows = 4;  // rows of a block of the render kernels' 32 x 4-thread form
 
 template <class T>
 struct Pt {
@@ -98,15 +98,18 @@ struct Slot {
     unsigned long long *h_sum = nullptr;  // pinned
 };
 
+// A render kernel of the module and its other forms (null if the module lacks them).
+struct RenderForms {
+    cu_function whole = nullptr, strip = nullptr, group = nullptr;
+};
+
 }  // namespace
 
 struct cu_serve_s {
     cu_engine engine = nullptr;
     cu_module module = nullptr;
-    cu_function main_f = nullptr, main_d = nullptr, adv_f = nullptr, adv_d = nullptr,
-                compose = nullptr, checksum = nullptr;
-    // the render kernels for 32 x 4-thread blocks (null if the module lacks them)
-    cu_function main_fs = nullptr, main_ds = nullptr, adv_fs = nullptr, adv_ds = nullptr;
+    RenderForms main_f, main_d, adv_f, adv_d;
+    cu_function compose = nullptr, checksum = nullptr;
     void *d_module_iters = nullptr;  // module symbol cu_iteration_slots
     cu_serve_config cfg{};
     std::vector<Slot> slots;
@@ -217,18 +220,20 @@ void launch_module(cu_function f, unsigned gx, unsigned gy, void **params, hipSt
           (std::string("hipModuleLaunchKernel ") + f->name).c_str());
 }
 
-// A render kernel over a W x H frame: its 32 x 4-thread form over ceil(W/32) x
-// ceil(H/4) blocks when the module has one (the same pixels and results), else
-// the reference's 32 x 32 blocks.
-void launch_render(cu_function f, cu_function strip, uint32_t W, uint32_t H, void **params,
+// A render kernel over a W x H frame: one of its forms (render_form.hpp) over
+// ceil(W/32) x ceil(H/4) blocks when the module has it (the same pixels and results),
+// else the reference's 32 x 32 blocks.
+void launch_render(const RenderForms &k, bool one_group, uint32_t W, uint32_t H, void **params,
                    hipStream_t st) {
     const unsigned gx = (W + kBlockDim - 1) / kBlockDim;
-    if (strip) {
-        check(hipModuleLaunchKernel(strip->function, gx, (H + kStripRows - 1) / kStripRows, 1,
-                                    kBlockDim, kStripRows, 1, 0, st, params, nullptr),
-              (std::string("hipModuleLaunchKernel ") + strip->name).c_str());
+    const cu_function form = one_group && k.group ? k.group : k.strip;
+    if (form) {
+        check(hipModuleLaunchKernel(form->function, gx, (H + kStripRows - 1) / kStripRows, 1,
+                                    kBlockDim, form == k.group ? kGroupTRows : kStripRows, 1, 0, st,
+                                    params, nullptr),
+              (std::string("hipModuleLaunchKernel ") + form->name).c_str());
     } else {
-        launch_module(f, gx, (H + kBlockDim - 1) / kBlockDim, params, st);
+        launch_module(k.whole, gx, (H + kBlockDim - 1) / kBlockDim, params, st);
     }
 }
 
@@ -262,6 +267,7 @@ void dispatch(cu_serve_s *s, Session &ss, Slot &sl, const Request &rq) {
         Rect<double> rd = rect;
         uint32_t maxit = r.max_iter;
         float max_ss = s->cfg.max_super_sampling;
+        const PlaneRect plane{rect.lbx, rect.lby, rect.rtx, rect.rty};
         const unsigned gx = (W + kBlockDim - 1) / kBlockDim, gy = (H + kBlockDim - 1) / kBlockDim;
         if (!ss.has_prev) {  // renderQuality: main kernel into the primary buffer
             void *out = ss.buf[ss.primary];
@@ -269,8 +275,8 @@ void dispatch(cu_serve_s *s, Session &ss, Slot &sl, const Request &rq) {
             uint32_t flags = CU_FLAG_ADAPTIVE_SS;
             void *params[] = {&out, &pitch, &size, fp32 ? (void *)&rf : (void *)&rd, &maxit,
                               &max_ss, &flags};
-            launch_render(fp32 ? s->main_f : s->main_d, fp32 ? s->main_fs : s->main_ds, W, H, params,
-                          st);
+            launch_render(fp32 ? s->main_f : s->main_d,
+                          one_group_waves(W, H, max_ss, false, plane, plane), W, H, params, st);
             path = 1;
         } else {  // renderFast: advanced kernel primary -> secondary, then swap
             void *in = ss.buf[ss.primary];
@@ -286,7 +292,10 @@ void dispatch(cu_serve_s *s, Session &ss, Slot &sl, const Request &rq) {
             void *params[] = {&out, &out_pitch, &size, fp32 ? (void *)&rf : (void *)&rd, &maxit,
                               &max_ss, &flags, fp32 ? (void *)&of : (void *)&od, &in, &in_pitch,
                               &focus};
-            launch_render(fp32 ? s->adv_f : s->adv_d, fp32 ? s->adv_fs : s->adv_ds, W, H, params, st);
+            launch_render(fp32 ? s->adv_f : s->adv_d,
+                          one_group_waves(W, H, max_ss, true, plane,
+                                          {od.lbx, od.lby, od.rtx, od.rty}),
+                          W, H, params, st);
             ss.primary = 1 - ss.primary;
             path = 0;
         }
@@ -453,14 +462,15 @@ int cu_serve_create(const char *kernels_dir, const cu_serve_config *cfg, cu_serv
         if (cu_engine_create(kernels_dir, &s->engine) != CU_OK) fail(CU_ERR_INITIALIZATION, cu_last_error());
         const std::string path = std::string(kernels_dir) + "/mandelbrot.hsaco";
         if (cu_module_load(path.c_str(), &s->module) != CU_OK) fail(CU_ERR_INITIALIZATION, cu_last_error());
-        s->main_f = module_fn(s->module, "fractalRenderMainFloat");
-        s->main_d = module_fn(s->module, "fractalRenderMainDouble");
-        s->adv_f = module_fn(s->module, "fractalRenderAdvancedFloat");
-        s->adv_d = module_fn(s->module, "fractalRenderAdvancedDouble");
-        s->main_fs = module_fn_if(s->module, "fractalRenderMainFloatStrip");
-        s->main_ds = module_fn_if(s->module, "fractalRenderMainDoubleStrip");
-        s->adv_fs = module_fn_if(s->module, "fractalRenderAdvancedFloatStrip");
-        s->adv_ds = module_fn_if(s->module, "fractalRenderAdvancedDoubleStrip");
+        const auto forms = [&](const std::string &name) {
+            return RenderForms{module_fn(s->module, name.c_str()),
+                               module_fn_if(s->module, (name + "Strip").c_str()),
+                               module_fn_if(s->module, (name + "Group").c_str())};
+        };
+        s->main_f = forms("fractalRenderMainFloat");
+        s->main_d = forms("fractalRenderMainDouble");
+        s->adv_f = forms("fractalRenderAdvancedFloat");
+        s->adv_d = forms("fractalRenderAdvancedDouble");
         s->compose = module_fn(s->module, "compose");
         s->checksum = function(s->engine, "checksumU32");
         size_t bytes = 0;

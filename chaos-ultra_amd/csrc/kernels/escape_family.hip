@@ -278,8 +278,9 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
         }
         if ((run | ended) == 0) break;
 
-        cu::run_blocks<Real, K, kFused, false>(o, run, failed, ended, exhausted ? run | ended : ~0ull,
-                                        refill, max_iter, bsq);
+        cu::run_blocks<Real, K, kFused, false>(o, run, failed, ended,
+                                               exhausted ? run | ended : ~0ull, refill, max_iter,
+                                               bsq);
 
         // ---- pending lanes: locate the escape or run checked steps, finish the sample ----
         bool another = false;

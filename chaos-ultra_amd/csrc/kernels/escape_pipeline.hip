@@ -106,7 +106,8 @@ __device__ __forceinline__ bool run_lanes(const PipeArgs &a, bool active, Real x
     o.template begin<K>(max_iter, cu::kCycleFirstMixed);
     uint64_t run = cu::ballot(active && blocks && max_iter - i >= (uint)K);
     uint64_t failed = 0, ended = cu::ballot(active) & ~run;
-    cu::run_blocks<Real, K, kFused, true>(o, run, failed, ended, ~0ull, 64u - a.handoff, max_iter, bsq);
+    cu::run_blocks<Real, K, kFused, true>(o, run, failed, ended, ~0ull, 64u - a.handoff, max_iter,
+                                          bsq);
     count = 0;
     smooth = 0;
     const bool done = cu::in_mask(failed | ended);
@@ -415,8 +416,9 @@ __device__ void drain(const PipeArgs a, const Straggler<Real> *queue, const uint
         if ((run | ended) == 0) break;
 
         // ---- unchecked blocks until enough lanes wait ----
-        cu::run_blocks<Real, K, kFused, false>(o, run, failed, ended, exhausted ? run | ended : ~0ull,
-                                        refill, max_iter, bsq);
+        cu::run_blocks<Real, K, kFused, false>(o, run, failed, ended,
+                                               exhausted ? run | ended : ~0ull, refill, max_iter,
+                                               bsq);
 
         // ---- pending lanes finish their sample ----
         if (cu::in_mask(failed | ended)) {

@@ -58,14 +58,25 @@ constexpr uint kZoomingInFlag = 1u << 5;
 // spreads the blocks a CU receives over the frame; a tile and its vote groups
 // are the reference's, only the block that computes them differs.  A block of
 // 32 x 4 threads (the *Strip kernels) covers 32 x 4 pixels the same way: the
-// same 8x4 rectangles, and the same two of them in each wave.
-__device__ __forceinline__ Point<uint> image_indexes() {
-    const uint t = threadIdx.x + threadIdx.y * 32u;
-    const uint warp = t >> 5, lane = t & 31u;
+// same 8x4 rectangles, and the same two of them in each wave (kGroups).  With one
+// rectangle a wave (the *Group kernels, 32 x 8 threads for the same pixels) the
+// upper 32 lanes own no pixel and only iterate orbits of the others'.
+template <uint kGroups>
+__device__ __forceinline__ Point<uint> image_indexes_at(uint t) {  // flat thread index t
+    const uint warp = kGroups == 2u ? t >> 5 : t >> 6, lane = t & 31u;
     Point<uint> p;
     p.x = cu::skewed_block_x() * 32u + (warp & 3u) * 8u + (lane >> 4) * 4u + (lane & 3u);
-    p.y = blockIdx.y * blockDim.y + (warp >> 2) * 4u + ((lane >> 2) & 3u);
+    p.y = blockIdx.y * (blockDim.y * kGroups / 2u) + (warp >> 2) * 4u + ((lane >> 2) & 3u);
     return p;
+}
+template <uint kGroups>
+__device__ __forceinline__ Point<uint> image_indexes() {
+    return image_indexes_at<kGroups>(threadIdx.x + threadIdx.y * 32u);
+}
+// Whether this lane owns pixel p of an image.
+template <uint kGroups>
+__device__ __forceinline__ bool owns(Point<uint> p, Point<uint> size) {
+    return p.x < size.x && p.y < size.y && (kGroups == 2u || cu::lane_id() < 32u);
 }
 
 __device__ __forceinline__ pixel_info_t *pixel_at(pixel_info_t *base, long pitch, uint x, uint y) {
@@ -132,15 +143,6 @@ __device__ __forceinline__ float dispersion(const float (&samples)[kAdaptiveThre
     }
     variance /= (n - 1);
     return variance / mean;
-}
-
-// Pixel of flat thread index t of the block (getImageIndexes, :36-53).
-__device__ __forceinline__ Point<uint> image_indexes_at(uint t) {
-    const uint warp = t >> 5, lane = t & 31u;
-    Point<uint> p;
-    p.x = cu::skewed_block_x() * 32u + (warp & 3u) * 8u + (lane >> 4) * 4u + (lane & 3u);
-    p.y = blockIdx.y * blockDim.y + (warp >> 2) * 4u + ((lane >> 2) & 3u);
-    return p;
 }
 
 // Sample offsets of sample i of a pixel asked for sampleCountF samples (:105-117).
@@ -224,7 +226,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // view, FP32, maxIter 1600, 5 adaptive spp: 408 -> 290 us (392 without the cycle
 // test); a bounded Julia set at 1280x720 308 -> 90 us; the 4096^2 frame's view in
 // 4K, FP64, 4 spp 1572 -> 1547 us, its 1080p zoom frames 450 -> 392 us.
-template <class Real, bool kFused>
+template <class Real, bool kFused, uint kGroups>
 __device__ uint sample_the_fractal(WaveLds &lds, int site, Point<uint> grid, Rectangle<Real> image,
                                    uint max_iter, float &sample_count_f, bool adaptive,
                                    uint64_t &executed) {
@@ -354,7 +356,7 @@ __device__ uint sample_the_fractal(WaveLds &lds, int site, Point<uint> grid, Rec
                 const float orow_f = __shfl(per_row_f, (int)src, 64);
                 if (take) {
                     task = h;
-                    const Point<uint> op = image_indexes_at(wave_base + src);
+                    const Point<uint> op = image_indexes_at<kGroups>(wave_base + src);
                     Real dx, dy;
                     sample_offset<Real>(h >> 8, orow_f, dx, dy);
                     // c = leftTop + (1,-1) * (pixel + delta) * pixelSize  (:119-124)
@@ -369,8 +371,8 @@ __device__ uint sample_the_fractal(WaveLds &lds, int site, Point<uint> grid, Rec
         }
 
         // ---- unchecked blocks until kRefill lanes wait (idle ones count while work is left) ----
-        cu::run_blocks<Real, K, kFused, false>(o, run, failed, ended, more ? ~0ull : run | ended, kRefill,
-                                        max_iter, bsq);
+        cu::run_blocks<Real, K, kFused, false>(o, run, failed, ended, more ? ~0ull : run | ended,
+                                               kRefill, max_iter, bsq);
 
         // ---- finish the pending orbits and post their iteration counts ----
         if (cu::in_mask(failed | ended)) {
@@ -404,21 +406,23 @@ __device__ __forceinline__ bool fused_valid(Rectangle<Real> image, Point<uint> g
     }
 }
 
-template <class Real, uint kWaves>
+template <class Real, uint kWaves, uint kGroups>
 __device__ void render_main(pixel_info_t *out, long out_pitch, Point<uint> size,
                             Rectangle<Real> image, uint max_iter, float max_ss, uint flags) {
-    const Point<uint> idx = image_indexes();
-    const bool inside = idx.x < size.x && idx.y < size.y;
+    const Point<uint> idx = image_indexes<kGroups>();
+    const bool inside = owns<kGroups>(idx, size);
     float sample_count = max_ss;
     uint64_t executed = 0;
     __shared__ WaveLds lds_waves[kWaves];
     WaveLds &lds = lds_waves[(threadIdx.x + threadIdx.y * blockDim.x) >> 6];
     const bool adaptive = (flags & kAdaptiveFlag) != 0;
     const uint r = fused_valid<Real>(image, size)
-                       ? sample_the_fractal<Real, true>(lds, inside ? 1 : 0, size, image, max_iter,
-                                                        sample_count, adaptive, executed)
-                       : sample_the_fractal<Real, false>(lds, inside ? 1 : 0, size, image, max_iter,
-                                                         sample_count, adaptive, executed);
+                       ? sample_the_fractal<Real, true, kGroups>(lds, inside ? 1 : 0, size, image,
+                                                                 max_iter, sample_count, adaptive,
+                                                                 executed)
+                       : sample_the_fractal<Real, false, kGroups>(lds, inside ? 1 : 0, size, image,
+                                                                  max_iter, sample_count, adaptive,
+                                                                  executed);
     count_iterations(executed);
     if (inside) {
         pixel_info_t p;
@@ -494,13 +498,13 @@ __device__ __forceinline__ void foveation(Point<uint> pixel, Point<uint> focus, 
     }
 }
 
-template <class Real, uint kWaves>
+template <class Real, uint kWaves, uint kGroups>
 __device__ void render_advanced(pixel_info_t *out, long out_pitch, Point<uint> size,
                                 Rectangle<Real> image, uint max_iter, float max_ss, uint flags,
                                 Rectangle<Real> image_reused, const pixel_info_t *in,
                                 long in_pitch, Point<uint> focus) {
-    const Point<uint> idx = image_indexes();
-    const bool in_image = idx.x < size.x && idx.y < size.y;
+    const Point<uint> idx = image_indexes<kGroups>();
+    const bool in_image = owns<kGroups>(idx, size);
 
     float advised = max_ss;
     bool in_focus = false;
@@ -549,10 +553,10 @@ __device__ void render_advanced(pixel_info_t *out, long out_pitch, Point<uint> s
     WaveLds &lds = lds_waves[(threadIdx.x + threadIdx.y * blockDim.x) >> 6];
     const bool adaptive = (flags & kAdaptiveFlag) != 0;
     const uint r = fused_valid<Real>(image, size)
-                       ? sample_the_fractal<Real, true>(lds, site, size, image, max_iter,
-                                                        sample_count, adaptive, executed)
-                       : sample_the_fractal<Real, false>(lds, site, size, image, max_iter,
-                                                         sample_count, adaptive, executed);
+                       ? sample_the_fractal<Real, true, kGroups>(lds, site, size, image, max_iter,
+                                                                 sample_count, adaptive, executed)
+                       : sample_the_fractal<Real, false, kGroups>(
+                             lds, site, size, image, max_iter, sample_count, adaptive, executed);
     count_iterations(executed);
     if (site == 1) {  // :349-356
         const float samples = (float)r;
@@ -580,24 +584,24 @@ __device__ __forceinline__ uint colorize_sample_count(uint sample_count, uint fu
 
 extern "C" __global__ void init() {}
 
-#define CU_RENDER_KERNELS(SUFFIX, BOUNDS, BOUNDS_ADV_DOUBLE, WAVES)                               \
+#define CU_RENDER_KERNELS(SUFFIX, BOUNDS, BOUNDS_ADV_DOUBLE, WAVES, GROUPS)                         \
     extern "C" __global__ BOUNDS void fractalRenderMainFloat##SUFFIX(                               \
         pixel_info_t *output, long outputPitch, Point<uint> outputSize, Rectangle<float> image,     \
         uint maxIterations, float maxSuperSampling, uint flags) {                                   \
-        render_main<float, WAVES>(output, outputPitch, outputSize, image, maxIterations,            \
+        render_main<float, WAVES, GROUPS>(output, outputPitch, outputSize, image, maxIterations,    \
                                   maxSuperSampling, flags);                                         \
     }                                                                                               \
     extern "C" __global__ BOUNDS void fractalRenderMainDouble##SUFFIX(                              \
         pixel_info_t *output, long outputPitch, Point<uint> outputSize, Rectangle<double> image,    \
         uint maxIterations, float maxSuperSampling, uint flags) {                                   \
-        render_main<double, WAVES>(output, outputPitch, outputSize, image, maxIterations,           \
+        render_main<double, WAVES, GROUPS>(output, outputPitch, outputSize, image, maxIterations,   \
                                    maxSuperSampling, flags);                                        \
     }                                                                                               \
     extern "C" __global__ BOUNDS void fractalRenderAdvancedFloat##SUFFIX(                           \
         pixel_info_t *output, long outputPitch, Point<uint> outputSize, Rectangle<float> image,     \
         uint maxIterations, float maxSuperSampling, uint flags, Rectangle<float> imageReused,       \
         const pixel_info_t *input, long inputPitch, Point<uint> focus) {                            \
-        render_advanced<float, WAVES>(output, outputPitch, outputSize, image, maxIterations,        \
+        render_advanced<float, WAVES, GROUPS>(output, outputPitch, outputSize, image, maxIterations,\
                                       maxSuperSampling, flags, imageReused, input, inputPitch,      \
                                       focus);                                                       \
     }                                                                                               \
@@ -605,14 +609,14 @@ extern "C" __global__ void init() {}
         pixel_info_t *output, long outputPitch, Point<uint> outputSize, Rectangle<double> image,    \
         uint maxIterations, float maxSuperSampling, uint flags, Rectangle<double> imageReused,      \
         const pixel_info_t *input, long inputPitch, Point<uint> focus) {                            \
-        render_advanced<double, WAVES>(output, outputPitch, outputSize, image, maxIterations,       \
+        render_advanced<double, WAVES, GROUPS>(output, outputPitch, outputSize, image, maxIterations,\
                                        maxSuperSampling, flags, imageReused, input, inputPitch,     \
                                        focus);                                                      \
     }
 
 // The reference's kernels: 32 x 32-thread blocks over ceil(W/32) x ceil(H/32)
 // (CudaFractalRenderer.java:242-258), 16 waves and their LDS per block.
-CU_RENDER_KERNELS(, __launch_bounds__(1024), __launch_bounds__(1024), 16u)
+CU_RENDER_KERNELS(, __launch_bounds__(1024), __launch_bounds__(1024), 16u, 2u)
 
 // The same kernels for 32 x 4-thread blocks over ceil(W/32) x ceil(H/4), which
 // the renderer layer and the serving loop launch: the same pixels, vote groups
@@ -621,7 +625,12 @@ CU_RENDER_KERNELS(, __launch_bounds__(1024), __launch_bounds__(1024), 16u)
 // for 4 of them: about 3 waves per SIMD stay resident.  Blocks of 2 waves keep
 // the wave slots filled (14 blocks per CU, 136 KB of LDS).  The FP64 advanced
 // kernel needs 78 VGPRs: it is held to 6 waves per SIMD rather than spill.
-CU_RENDER_KERNELS(Strip, __launch_bounds__(128, 7), __launch_bounds__(128, 6), 2u)
+CU_RENDER_KERNELS(Strip, __launch_bounds__(128, 7), __launch_bounds__(128, 6), 2u, 2u)
+
+// One vote group a wave, 32 x 8-thread blocks over the same grid as *Strip, for launches
+// that wait for the waves with the most samples to run (when: host/render_form.hpp): its
+// 32 pixels' samples have 64 lanes, and what a wave runs one after the other halves.
+CU_RENDER_KERNELS(Group, __launch_bounds__(256, 7), __launch_bounds__(256, 6), 4u, 1u)
 
 // compose (fractalRendererGeneric.cu:455-475).  The palette is staged in LDS
 // (up to kPaletteLds entries; longer palettes are read from global memory) and

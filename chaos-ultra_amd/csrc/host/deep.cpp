@@ -404,6 +404,9 @@ int cu_deep_orbit(cu_deep d, void *host_out, uint32_t capacity_entries, uint32_t
         if ((uint64_t)M + 1 > capacity_entries) fail(CU_ERR_ILLEGAL_ARGUMENT, "capacity too small");
         check(hipMemcpy(host_out, d->d_orbit[0], ((size_t)M + 1) * d->entry_bytes,
                         hipMemcpyDeviceToHost), "hipMemcpy D2H");
+        // the fourth value of an entry is the pixel kernels' own
+        unsigned char *fourth = (unsigned char *)host_out + d->entry_bytes / 4 * 3;
+        for (size_t m = 0; m <= M; ++m) std::memset(fourth + m * d->entry_bytes, 0, d->entry_bytes / 4);
         *length = M;
     });
 }

@@ -89,8 +89,12 @@ __device__ __forceinline__ void dd_orbit_step(DD &x, DD &y, DD cx, DD cy) {
 
 template <class Real>
 struct alignas(4 * sizeof(Real)) OrbitEntry {
-    Real x, y, h, pad;  // Z_m and |Z_m|^2 / 2
+    Real x, y, h;  // Z_m and |Z_m|^2 / 2
+    Real quiet;    // 0, or where a block starts (m % kPlainSteps == 0) its quiet_bound
 };
+
+// Steps of the pixel kernels' blocks.
+constexpr int kPlainSteps = 32;
 
 // Pointers into LDS and global memory typed with their address spaces, so that
 // loads through them stay LDS or global (or scalar) loads: through untyped
@@ -107,7 +111,7 @@ __device__ __forceinline__ OrbitEntry<Real> load_entry(Ptr p) {
     e.x = p->x;
     e.y = p->y;
     e.h = p->h;
-    e.pad = 0;
+    e.quiet = 0;
     return e;
 }
 
@@ -150,7 +154,7 @@ __device__ uint orbit_entries(double cx_hi, double cx_lo, double cy_hi, double c
         e.x = (Real)x.hi;
         e.y = (Real)y.hi;
         e.h = (Real)(0.5 * mag);
-        e.pad = 0;
+        e.quiet = 0;
         orbit[at] = e;
         return mag < bailout_sq;
     };
@@ -226,7 +230,28 @@ __device__ void orbit_cycle(const OrbitEntry<Real> *orbit, uint M, uint &period,
     }
 }
 
-// One wave: its first lane computes the orbit, all look for the cycle.
+// The bound C with which no rebase test fires in the block of kPlainSteps steps from entry
+// m, whatever the lane, if (|d| + |dc|) C < 1 at its start.  While |d_j| <= |Z_j| / 4, a
+// step gives |d'| <= (2 |Z| + |Z| / 4) |d| + |dc|, so with E = |d| + |dc| at the start
+// |d_k| <= E U_k for U_0 = 1, U_k+1 = 2.25 |Z_k| U_k + 1; and at |d| <= |Z| / 4 the test,
+// Z.d < -|Z|^2 / 2, is far from firing.  C is the largest 4 U_k / |Z_k|.  The margins of 4 %
+// a step are many times the roundings of a step and of this sum, in FP32 too.  Where |Z| is
+// small (the orbit starts at 0) there is no bound.
+template <class Real>
+__device__ float quiet_bound(const OrbitEntry<Real> *orbit, uint m) {
+    float u = 1, c = 0;
+#pragma unroll 8
+    for (int k = 0; k < kPlainSteps; ++k) {
+        const float x = (float)orbit[m + k].x, y = (float)orbit[m + k].y;
+        const float z = sqrtf(x * x + y * y);
+        c = z > 1e-6f ? fmaxf(c, 4.16f * u / z) : __builtin_inff();
+        u = 2.35f * z * u + 1.04f;
+    }
+    return c;
+}
+
+// One wave: its first lane computes the orbit, all look for the cycle and for the blocks'
+// quiet bounds.
 template <class Real>
 __device__ void reference_orbit(double cx_hi, double cx_lo, double cy_hi, double cy_lo,
                                 uint max_iter, double bailout_sq, OrbitEntry<Real> *orbit,
@@ -239,6 +264,8 @@ __device__ void reference_orbit(double cx_hi, double cx_lo, double cy_hi, double
     const uint M = __builtin_amdgcn_readfirstlane(n);
     uint period = 0, start = 0;
     if (M == max_iter && M != 0) orbit_cycle<Real>(orbit, M, period, start);
+    for (uint b = threadIdx.x; b < M / kPlainSteps; b += 64)
+        orbit[b * kPlainSteps].quiet = (Real)quiet_bound<Real>(orbit, b * kPlainSteps);
     if (threadIdx.x == 0) *info = {M, period, start, 0};
 }
 
@@ -352,7 +379,10 @@ __device__ __forceinline__ int checked_step(const OrbitView<Real> &Z, uint M, Re
 // time, one scalar load for two FP64 or four FP32 ones: in 1e-10 and 1e-20 frames with
 // FP64 deltas 3 % less time than with two loads an entry, 1 to 3 % at 1e-6 (the other
 // waves cover the loads' latency; asking one group ahead was slower by a tenth).
-template <class Real, int K>
+//
+// Without kTest it leaves the tests out and returns 0, for blocks in which none can fire
+// (quiet_bound): 6 VALU instructions a step against 9.
+template <class Real, int K, bool kTest>
 __device__ __forceinline__ uint64_t unchecked_block(global_ptr<OrbitEntry<Real>> zp, Real &dx,
                                                     Real &dy, Real dcx, Real dcy) {
     constexpr int kTogether = 64 / (int)sizeof(OrbitEntry<Real>);
@@ -364,7 +394,7 @@ __device__ __forceinline__ uint64_t unchecked_block(global_ptr<OrbitEntry<Real>>
 #pragma unroll
         for (int j = 0; j < kTogether; ++j) {
             const Real x = z[4 * j], y = z[4 * j + 1], h = z[4 * j + 2];
-            flagged |= cu::ballot(rebase_test(x, y, h, dx, dy));
+            if constexpr (kTest) flagged |= cu::ballot(rebase_test(x, y, h, dx, dy));
             const Real ax = cu::fma_r((Real)2, x, dx);
             const Real ay = cu::fma_r((Real)2, y, dy);
             const Real ndx = cu::fma_r(ax, dx, cu::fma_r(-ay, dy, dcx));
@@ -450,12 +480,12 @@ __device__ __forceinline__ uint64_t rebasing_block(Ptr orbit, uint M, const Orbi
 //
 // Bound by VALU issue, and by the longest waves once the others have ended; 1920x1080,
 // without the reference orbit's time, FP32 / FP64 deltas: 1e-10 (each pixel rebases on
-// its own) 1.50 / 2.24 -> 1.07 / 1.83 ms, a shallow frame of width 1 2.85 / 3.80 ->
-// 0.43 / 0.71 ms (0.70 / 1.15 without the cycles along the reference's), 1e-20 (few
-// rebases) 1.20 / 2.03 -> 1.15 / 1.87 ms; before, a block stopped for the whole wave at
-// its first rebase, and each escape was replayed as it came, 32 checked steps for one
-// lane.  1e-6, three quarters interior, 18.7 / 32.7 -> 8.8 / 19.1 ms, 11.0 / 22.0 of it
-// by the cycle test.
+// its own) 1.50 / 2.24 -> 1.00 / 1.73 ms, a shallow frame of width 1 2.85 / 3.80 ->
+// 0.44 / 0.73 ms (0.70 / 1.15 without the cycles along the reference's), 1e-20 (few
+// rebases) 1.20 / 2.03 -> 0.80 / 1.39 ms (1.14 / 1.88 with the tests in every block);
+// before, a block stopped for the whole wave at its first rebase, and each escape was
+// replayed as it came, 32 checked steps for one lane.  1e-6, three quarters interior,
+// 18.7 / 32.7 -> 8.8 / 19.1 ms, 11.0 / 22.0 of it by the cycle test.
 template <class Real, int K>
 __device__ int perturb_pixel(const OrbitView<Real> &Z, const OrbitInfo &info, Real dcx,
                              Real dcy, uint max_iter, Real bsq, bool rebase, Real geps,
@@ -476,6 +506,8 @@ __device__ int perturb_pixel(const OrbitView<Real> &Z, const OrbitInfo &info, Re
         uint64_t along = 0;              // lanes that hold their delta on the reference's cycle
         uint due = 0;                    // iteration count at which theirs is looked for
         const uint stride = info.period * ((uint)K >> __builtin_ctz(info.period | (uint)K));
+        uint bounded = 0;                // entry whose quiet_bound, if it has one, is loaded
+        Real quiet = __builtin_inff();   // (ahead of its use: a load here would be waited for)
         uint streak = 0;                 // consecutive blocks rerun for a rebase
         const OrbitEntry<Real> z1 = load_entry<Real>(Z.global + min(1u, M));
         while (run != 0 && max_iter - n >= (uint)K) {
@@ -494,9 +526,21 @@ __device__ int perturb_pixel(const OrbitView<Real> &Z, const OrbitInfo &info, Re
             bool plain = same && !near && streak < 2;
             if (plain) {
                 const Real bx = dx, by = dy;
-                plain = (unchecked_block<Real, K>(Z.global + mu, dx, dy, dcx, dcy) & run) == 0;
+                bool none = false;  // whether no test can fire in this block
+                if (mu == bounded && mu % (uint)K == 0) {
+                    const Real size = __builtin_fabs(dx) + __builtin_fabs(dy) +
+                                      (__builtin_fabs(dcx) + __builtin_fabs(dcy));
+                    none = (run & ~cu::ballot(size * quiet < 1)) == 0;
+                }
+                if (none)
+                    unchecked_block<Real, K, false>(Z.global + mu, dx, dy, dcx, dcy);
+                else
+                    plain = (unchecked_block<Real, K, true>(Z.global + mu, dx, dy, dcx, dcy) &
+                             run) == 0;
                 if (plain) {
                     e = load_entry<Real>(Z.global + (mu + (uint)K));
+                    bounded = mu + (uint)K;
+                    quiet = Z.global[bounded].quiet;
                     m += (uint)K;
                     streak = 0;
                 } else {
@@ -551,7 +595,7 @@ __device__ int perturb_pixel(const OrbitView<Real> &Z, const OrbitInfo &info, Re
             }
             if (n >= hold) {
                 cu::seldom();
-                along = info.period != 0 ? run & cu::ballot(m >= info.start) : 0;
+                along = stride != 0 ? run & cu::ballot(m >= info.start) : 0;
                 if (cu::in_mask(along))
                     held.take(dx, dy);
                 else
@@ -603,6 +647,7 @@ __device__ __forceinline__ void deep_pixel_coords(uint &px, uint &py) {
 //   FP64: 4 x 2 waves (32 x 16 pixels, 512 threads), 40 KB = 1280 entries, 4 blocks per CU
 template <class Real, int K, uint WX, uint WY, uint LdsBytes>
 __device__ void perturb_frame(const DeepArgs a, const OrbitEntry<Real> *__restrict__ orbit) {
+    static_assert(K == kPlainSteps, "the orbit's quiet bounds are for blocks of that length");
     __shared__ OrbitEntry<Real> lds[LdsBytes / sizeof(OrbitEntry<Real>)];
     const OrbitInfo info = *a.info;
     const uint staged = min(info.last + 1u, LdsBytes / (uint)sizeof(OrbitEntry<Real>));

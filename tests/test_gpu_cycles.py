@@ -199,3 +199,17 @@ def test_perturbation_along_a_periodic_reference(gpu, engine, oracle, centre, wi
         assert np.array_equal(frame.counts().ravel(), wc)
         assert report.iterations == wit
     frame.close()
+
+
+# frames whose deltas grow from far below the reference's values to rebases and escapes, so that
+# their blocks run without tests, then with them; the reference of the second comes close to 0
+# every third step, the fourth's limit ends inside the first phase
+@pytest.mark.parametrize("centre,width,limit", [
+    ((-0.743643887037151, 0.131825904205330), 1e-12, 4001),
+    ((-1.7548776662466927, 0.0), 1e-3, 1501), ((-1.7548776662466927, 1e-9), 1e-9, 1501),
+    ((-0.743643887037151, 0.131825904205330), 1e-25, 1000), ((0.0, 1.0), 1e-10, 700),
+    ((0.2501, 0.0), 1e-5, 999)])
+@pytest.mark.parametrize("method", [32, 64])
+def test_perturbation_blocks_without_tests(gpu, engine, oracle, centre, width, limit, method):
+    """Blocks in which no rebase test can fire leave them out, with the checked loop's result."""
+    deep_case(gpu, engine, oracle, gpu.make_deep(*centre, width, 45, 27, limit, 256.0), method)

@@ -130,54 +130,77 @@ struct OrbitView {
     }
 };
 
-// Entries 0 .. M of the orbit of C and M, the first index whose |Z|^2 fails the bailout
+// A state of the orbit where its entry goes: the leading parts of Z_m, in FP64.
+typedef double OrbitState __attribute__((ext_vector_type(2), may_alias));
+
+// States 0 .. M of the orbit of C, and M, the first index whose |Z|^2 fails the bailout
 // test, or max_iter.
 //
 // One lane's serial chain.  Alone on its SIMD it issues an instruction about every 5
 // cycles, dependent or not, and a taken branch costs it about 30, so what counts is
-// instructions and branches: kOrbitRun steps run without a test, each storing its entry,
-// and when a test among theirs failed they are taken again one by one from their start
-// (the entries stored past M are not read, and lie within the max_iter + 1 there are).
+// instructions and branches: kOrbitRun steps run without a test, each storing its state,
+// and when the last one's end fails the test they are taken again one by one from their
+// start (escape is permanent: bailout_sq >= 4, |C| <= 2; what is stored past M is not read,
+// and lies within the max_iter + 1 entries there are).  Entries are made of the states
+// afterwards, by the whole wave: 3088 of them 0.37 -> 0.32 ms, against a test and the
+// entry's |Z|^2 and conversions in every step.
 constexpr uint kOrbitRun = 8;
 
 template <class Real>
-__device__ uint orbit_entries(double cx_hi, double cx_lo, double cy_hi, double cy_lo,
-                              uint max_iter, double bailout_sq, OrbitEntry<Real> *orbit) {
+__device__ uint orbit_states(double cx_hi, double cx_lo, double cy_hi, double cy_lo,
+                             uint max_iter, double bailout_sq, OrbitEntry<Real> *orbit) {
     const DD cx{cx_hi, cx_lo}, cy{cy_hi, cy_lo};
     DD x{0.0, 0.0}, y{0.0, 0.0};
     uint n = 0;
-    auto store = [&](uint at) {  // entry `at`; whether the orbit goes on
+    auto store = [&](uint at) { *(OrbitState *)(orbit + at) = OrbitState{x.hi, y.hi}; };
+    auto inside = [&] {
         const double x2 = x.hi * x.hi;
         const double y2 = y.hi * y.hi;
-        const double mag = x2 + y2;
-        OrbitEntry<Real> e;
-        e.x = (Real)x.hi;
-        e.y = (Real)y.hi;
-        e.h = (Real)(0.5 * mag);
-        e.quiet = 0;
-        orbit[at] = e;
-        return mag < bailout_sq;
+        return x2 + y2 < bailout_sq;
     };
     while (max_iter - n >= kOrbitRun) {
         const DD x0 = x, y0 = y;
-        bool inside = true;
 #pragma unroll
         for (uint k = 0; k < kOrbitRun; ++k) {
-            inside &= store(n + k);
+            store(n + k);
             dd_orbit_step(x, y, cx, cy);
         }
-        if (!inside) {
+        if (!inside()) {
             x = x0;
             y = y0;
             break;
         }
         n += kOrbitRun;
     }
-    while (store(n) && n != max_iter) {
+    for (;;) {
+        store(n);
+        if (!inside() || n == max_iter) return n;
         dd_orbit_step(x, y, cx, cy);
         ++n;
     }
-    return n;
+}
+
+// The entries of states 0 .. M, by one wave.
+template <class Real>
+__device__ void orbit_entries(OrbitEntry<Real> *orbit, uint M) {
+    constexpr uint kTogether = 8;
+    for (uint from = threadIdx.x; from <= M; from += 64 * kTogether) {
+        OrbitState z[kTogether];
+#pragma unroll
+        for (uint j = 0; j < kTogether; ++j)
+            z[j] = *(const OrbitState *)(orbit + min(from + 64 * j, M));
+#pragma unroll
+        for (uint j = 0; j < kTogether; ++j) {
+            const double x2 = z[j].x * z[j].x;
+            const double y2 = z[j].y * z[j].y;
+            OrbitEntry<Real> e;
+            e.x = (Real)z[j].x;
+            e.y = (Real)z[j].y;
+            e.h = (Real)(0.5 * (x2 + y2));
+            e.quiet = 0;
+            if (from + 64 * j <= M) orbit[from + 64 * j] = e;
+        }
+    }
 }
 
 // The reference orbit as the pixel kernels need it beside its entries: the index of the
@@ -259,9 +282,11 @@ __device__ void reference_orbit(double cx_hi, double cx_lo, double cy_hi, double
     if (blockIdx.x != 0) return;
     uint n = 0;
     if (threadIdx.x == 0)
-        n = orbit_entries<Real>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit);
+        n = orbit_states<Real>(cx_hi, cx_lo, cy_hi, cy_lo, max_iter, bailout_sq, orbit);
     __syncthreads();
     const uint M = __builtin_amdgcn_readfirstlane(n);
+    orbit_entries<Real>(orbit, M);
+    __syncthreads();
     uint period = 0, start = 0;
     if (M == max_iter && M != 0) orbit_cycle<Real>(orbit, M, period, start);
     for (uint b = threadIdx.x; b < M / kPlainSteps; b += 64)

@@ -213,3 +213,27 @@ def test_perturbation_along_a_periodic_reference(gpu, engine, oracle, centre, wi
 def test_perturbation_blocks_without_tests(gpu, engine, oracle, centre, width, limit, method):
     """Blocks in which no rebase test can fire leave them out, with the checked loop's result."""
     deep_case(gpu, engine, oracle, gpu.make_deep(*centre, width, 45, 27, limit, 256.0), method)
+
+
+# a batch's queue order: by depth up to 256 tiles, above as they come; ties, one pixel, tiles of a row
+@pytest.mark.parametrize("n", [1, 2, 3, 64, 255, 256, 257, 700])
+def test_persistent_kernel_order_of_tiles(gpu, engine, oracle, n):
+    """Every tile's pixels land in its own place, whatever the order the queue takes them in."""
+    import importlib
+    at = importlib.import_module("chaos-ultra_amd.autotune")
+    rng = np.random.default_rng(n)
+    views = sorted(VIEWS)
+    tiles = [tile_of(gpu, views[rng.integers(len(views))], int(rng.choice([1, 40, 40, 333, 700, 701])),
+                     1, size=(int(rng.integers(1, 14)), int(rng.integers(1, 7)))) for _ in range(n)]
+    batch = at.PersistentBatch(gpu, tiles, 64)
+    batch.render(engine, gpu.Tune(16, 8, 64, 16))
+    gpu.synchronize()
+    counts, smooth = batch.counts.download(np.uint32), batch.smooth.download(np.float64)
+    total, offset = 0, 0
+    for t in tiles:
+        m = t.width * t.height
+        wc, ws, wit = oracle.escape_tile(t, 64)
+        same((counts[offset:offset + m], smooth[offset:offset + m], wit), (wc, ws, wit))
+        total += wit
+        offset += m
+    assert batch.iters.total() == total

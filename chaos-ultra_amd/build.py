@@ -113,9 +113,16 @@ def build_oracle() -> None:
     _run(["make", "-s", "-C", os.path.join(ROOT, "oracle")])
 
 
+def build_test_module() -> None:
+    """A module with the reference's kernels only (test infrastructure)."""
+    _run([_hipcc(), *HIP_FLAGS, "--genco", "plain_module.hip", "-o", "mandelbrot.hsaco"],
+         cwd=os.path.join(ROOT, "tests", "modules"))
+
+
 def build_all() -> None:
-    with ThreadPoolExecutor(max_workers=3) as ex:
-        futs = [ex.submit(build_modules), ex.submit(build_library), ex.submit(build_oracle)]
+    with ThreadPoolExecutor(max_workers=4) as ex:
+        futs = [ex.submit(build_modules), ex.submit(build_library), ex.submit(build_oracle),
+                ex.submit(build_test_module)]
         for f in futs:
             f.result()
     build_replay()

@@ -34,7 +34,6 @@ std::mutex g_mutex;
 bool g_debug_mode = false;  // -Ddebug=true (util/JavaHelpers.java:12,25-27)
 
 constexpr int kBlockDim = 32;          // CudaFractalRenderer.java:36-37
-constexpr int kComposeRows = 8;        // rows of a compose block; it strides over the other 24
 constexpr int kMaxGridDim = 65536 - 1;  // CudaFractalRenderer.java:34
 constexpr int kDefaultUnderSamplingLevel = 4;
 constexpr size_t kPixelInfoBytes = 16;  // SIZEOF_PIXEL_INFO_T (4) x 4 bytes
@@ -638,7 +637,8 @@ class Renderer {
             float max_ss = logger ? logger->max_super_sampling : 1.f;
             void *params[] = {&main, &main_pitch, &bcg, &bcg_pitch, &output_, &w, &h,
                               &palette_, &plen, &max_ss};
-            int rc = cu_launch_kernel(compose_, gx, gy, 1, kBlockDim, kComposeRows, 1, 0, params);
+            int rc = cu_launch_kernel(compose_, gx, gy, 1, kBlockDim, compose_rows(main_d_.strip != nullptr),
+                                      1, 0, params);
             if (rc == CU_OK) rc = cu_ctx_synchronize();
             if (rc != CU_OK) {
                 log_error(logger, std::string("Error just after launching a kernel:") + cu_last_error());

@@ -48,11 +48,6 @@ namespace {
 
 constexpr uint32_t kMaxSlots = 16;
 constexpr int kBlockDim = 32;  // reference launch geometry (CudaFractalRenderer.java:36-37)
-// Rows of a compose block, on the reference's grid: its threads stride over the other
-// rows of their 32.  A 1024-thread block only starts on a CU with 16 free wave slots,
-// which the other sessions' renders leave late: beside them compose took 207 us a frame
-// on average, 5 us alone.
-constexpr int kComposeRows = 8;
 
 template <class T>
 struct Pt {
@@ -309,8 +304,9 @@ void dispatch(cu_serve_s *s, Session &ss, Slot &sl, const Request &rq) {
         uint32_t w32 = W, h32 = H;
         void *cparams[] = {&main, &main_pitch, &bcg, &bcg_pitch, &rgba, &w32, &h32, &pal, &plen,
                            &max_ss};
-        check(hipModuleLaunchKernel(s->compose->function, gx, gy, 1, kBlockDim, kComposeRows, 1, 0,
-                                    st, cparams, nullptr),
+        check(hipModuleLaunchKernel(s->compose->function, gx, gy, 1, kBlockDim,
+                                    compose_rows(s->main_d.strip != nullptr), 1, 0, st, cparams,
+                                    nullptr),
               "hipModuleLaunchKernel compose");
         ss.has_prev = true;
         ss.prev = rect;

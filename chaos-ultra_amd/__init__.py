@@ -79,7 +79,7 @@ class DeviceBuffer:
     def download(self, dtype, count: int | None = None) -> np.ndarray:
         dtype = np.dtype(dtype)
         n = self.nbytes // dtype.itemsize if count is None else int(count)
-        out = _read_back.empty(n, dtype)
+        out = np.empty(n, dtype=dtype)
         abi.call("cu_memcpy_dtoh", out.ctypes.data_as(C.c_void_p), self.ptr, C.c_size_t(out.nbytes))
         return out
 
@@ -131,13 +131,14 @@ class HostBuffer:
 
 
 class _ReadBack:
-    """Arrays for reading device memory back, in page-locked memory: the copy then runs
-    at the link's rate instead of through the runtime's staging buffers into pages that
-    fault as they are touched (8.3 MB, a 1920x1080 image: 154 us against 466; 1 MB: 27
-    against 429).  An array owns its block until it and every view of it are gone; the
-    block then waits for the next array of its size class, unless CACHED bytes wait
-    already.  With LENT bytes in arrays that are still alive, and for small reads,
-    arrays are ordinary ones.  Any thread may ask, and any may drop an array."""
+    """Arrays for reading images back from the device, in page-locked memory: the copy
+    then runs at the link's rate instead of through the runtime's staging buffers into
+    pages that fault as they are touched (8.3 MB, a 1920x1080 image: 154 us against 466; 1 MB:
+    27 against 429).  An array owns its block until it and every view of it are gone; the
+    block then waits for the next array of its size class, unless CACHED bytes wait already.  With LENT bytes in arrays that are still alive,
+    and for small reads, arrays are ordinary ones.  Any thread may ask, and any may drop
+    an array.  numpy does not count such an array's memory as its own (in-place resize is
+    refused), so only entry points that return a view (an image's rows) use it."""
 
     SMALL, CACHED, LENT = 64 << 10, 256 << 20, 1 << 30
 
@@ -483,13 +484,13 @@ class Frame:
         abi.call("cu_frame_replay", self.handle, stream.handle if stream else None)
 
     def counts(self) -> np.ndarray:
-        out = _read_back.empty(self.total_pixels, np.uint32)
+        out = np.empty(self.total_pixels, dtype=np.uint32)
         abi.call("cu_memcpy_dtoh", out.ctypes.data_as(C.c_void_p), C.c_void_p(self.d_counts),
                  C.c_size_t(out.nbytes))
         return out
 
     def smooth(self) -> np.ndarray:
-        out = _read_back.empty(self.total_pixels, np.float64)
+        out = np.empty(self.total_pixels, dtype=np.float64)
         abi.call("cu_memcpy_dtoh", out.ctypes.data_as(C.c_void_p), C.c_void_p(self.d_smooth),
                  C.c_size_t(out.nbytes))
         return out

@@ -1,0 +1,50 @@
+"""Arrays read back from the device, with the copies and the page-locked allocation
+replaced by host stand-ins: which entry points return arrays that own their memory."""
+import ctypes as C
+import importlib
+import mmap
+
+import numpy as np
+import pytest
+
+
+@pytest.fixture
+def pkg(monkeypatch):
+    """The package with cu_host_alloc, cu_host_free and cu_memcpy_dtoh (which fills with
+    0x01 bytes) on the host."""
+    pkg = importlib.import_module("chaos-ultra_amd")
+    blocks = {}
+
+    def call(name, *args):
+        if name == "cu_host_alloc":
+            m = mmap.mmap(-1, args[1].value)
+            address = C.addressof(C.c_char.from_buffer(m))
+            blocks[address] = m
+            C.cast(args[0], C.POINTER(C.c_void_p))[0] = address
+        elif name == "cu_host_free":
+            del blocks[args[0].value]
+        else:
+            assert name == "cu_memcpy_dtoh"
+            C.memset(args[0], 1, args[2].value)
+
+    monkeypatch.setattr(pkg.abi, "call", call)
+    monkeypatch.setattr(pkg, "_read_back", pkg._ReadBack())
+    return pkg
+
+
+def made(cls, **fields):
+    thing = cls.__new__(cls)
+    thing.__dict__.update(fields)
+    return thing
+
+
+@pytest.mark.parametrize("words", [0, 100, 100_000, 2_000_000])
+def test_flat_arrays_own_their_memory(pkg, words):
+    """They can be resized in place, as any array that numpy allocated."""
+    buffer = made(pkg.DeviceBuffer, nbytes=4 * words, ptr=C.c_void_p())
+    frame = made(pkg.Frame, total_pixels=words, d_counts=0, d_smooth=0, handle=None)
+    for a in (buffer.download(np.uint32), buffer.download(np.uint8, 3 * words), frame.counts(),
+              frame.smooth()):
+        assert a.flags.owndata and a.flags.writeable and (a.view(np.uint8) == 1).all()
+        a.resize(a.size + 5, refcheck=False)
+        assert not a[-5:].any()

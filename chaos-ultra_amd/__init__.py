@@ -133,14 +133,19 @@ class HostBuffer:
 class _ReadBack:
     """Arrays for reading images back from the device, in page-locked memory: the copy
     then runs at the link's rate instead of through the runtime's staging buffers into
-    pages that fault as they are touched (8.3 MB, a 1920x1080 image: 154 us against 466; 1 MB:
-    27 against 429).  An array owns its block until it and every view of it are gone; the
-    block then waits for the next array of its size class, unless CACHED bytes wait already.  With LENT bytes in arrays that are still alive,
+    pages that fault as they are touched.  An array owns its block until it and every
+    view of it are gone; the block then waits for the next array of its size class,
+    unless CACHED bytes wait already.  With LENT bytes in arrays that are still alive,
     and for small reads, arrays are ordinary ones.  Any thread may ask, and any may drop
     an array.  numpy does not count such an array's memory as its own (in-place resize is
-    refused), so only entry points that return a view (an image's rows) use it."""
+    refused), so only entry points that return a view (an image's rows) use it.
 
-    SMALL, CACHED, LENT = 64 << 10, 256 << 20, 1 << 30
+    Ordinary against page-locked, us, where the program drops each array before the next
+    but one, and where it keeps them all (a block is then page-locked for each): 2 MB
+    122 -> 49, 506 -> 110; 8.3 MB (a 1920x1080 image) 456 -> 159, 1119 -> 263; at 384 KB
+    28 -> 20, 78 -> 78, and below that keeping them costs more."""
+
+    SMALL, CACHED, LENT = 384 << 10, 256 << 20, 1 << 30
 
     def __init__(self):
         # reentrant: dropping an array, in this thread too, may run while it is held

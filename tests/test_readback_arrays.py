@@ -48,3 +48,11 @@ def test_flat_arrays_own_their_memory(pkg, words):
         assert a.flags.owndata and a.flags.writeable and (a.view(np.uint8) == 1).all()
         a.resize(a.size + 5, refcheck=False)
         assert not a[-5:].any()
+
+
+@pytest.mark.parametrize("kilobytes,locked", [(64, False), (383, False), (384, True), (8100, True)])
+def test_small_images_are_ordinary_arrays(pkg, kilobytes, locked):
+    """Page-locking a block for an image that is kept only pays from 384 KB on."""
+    image = pkg._read_back.empty(256 * kilobytes, np.uint32)
+    assert image.flags.owndata != locked
+    assert (pkg._read_back._lent > 0) == locked

@@ -20,7 +20,6 @@
 namespace {
 
 constexpr uint kMaxLdsTiles = 1024;
-constexpr uint kMaxSortedTiles = 256;
 constexpr uint kPaletteLds = 4096;
 
 // Start sample `sample_id` = (py * width + px) * spp + s of tile t (pixel (px, py)):
@@ -172,53 +171,184 @@ __device__ void escape_tile_samples(const cu_tile_desc &t, double smooth_c, uint
 // Bound by VALU issue, then by the longest orbits at the end (a lone wave takes about
 // 17 ns a step, so 65536 of them 1.1 ms).  Batches of 32 and 24 uneven tiles, FP64,
 // tune 32/32/256/16: 7.7 -> 2.8 and 10.0 -> 2.2 ms (1.8e10 and 2.3e10 loop iterations)
-// with the cycle test, scalar lane masks and cursor (106 VGPRs against 115 with a
-// cursor the compiler kept per lane) and one resident set of waves; 32 tiles in FP32
+// with the cycle test, scalar lane masks and cursor and one resident set of waves (98
+// VGPRs, four blocks per CU); 32 tiles in FP32
 // 9.4 -> 1.8 ms.  Giving waves with old orbits issue priority (s_setprio) made no
 // batch faster and frames' tails up to 8 % slower.
+// A grab of the queue is of at least this many steps, at its tile's max_iter (as far as
+// `chunk` allows).  The counter takes an atomic every 13 ns, so 4096 waves must not come more
+// often than every 50 us, and pixels seldom run to max_iter.  With 64-pixel grabs at every
+// depth and with these: 16 tiles of 256^2, maxIter 50, 212 / 41 us, one of 1024^2, maxIter
+// 1000, 242 / 118, the headline frame's view there, maxIter 5000, 307 / 200; the other way, 1000
+// tiles of 8 to 40 pixels a side, maxIter 256 to 1024, 260 / 346.  Four times as many steps
+// leave waves with late deep grabs: 256 tiles of 50 to 200 pixels a side, maxIter 256 to
+// 65536, FP32, 5.0 -> 7.2 ms; half and twice as many are even.
+constexpr uint kGrabSteps = 1024u << 10;
+
+// From this max_iter on, batches that the waves' first grabs cover are put in order too (a
+// deep wave beside another on its SIMD takes twice as long; the first of the order go to
+// SIMDs of their own) and spread over half of the waves: 32 tiles of 8 to 97 pixels a side
+// 0.82 -> 0.69 ms.  Shallower ones are spread over all of them (maxIter up to 1024, 400
+// tiles of 8 to 40 pixels a side 211 -> 169 us) and not worth the order's time.
+constexpr uint kOrderDepth = 4096;
+
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Classes of max_iter, the deepest first: two to an octave, a lane of a wave each.
+__device__ __forceinline__ uint depth_class(uint depth) {
+    depth = max(depth, 1u);
+    const uint octave = 31u - __clz(depth);
+    return 63u - (2u * octave + (octave ? (depth >> (octave - 1)) & 1u : 0u));
+}
+
+// The queue's order of n tiles, by a block's four waves: from the deepest class of max_iter
+// down, so that the longest orbits do not start last, in a class as they come (24 batches
+// of 32 tiles of very different depth, 3.9 -> 3.2 ms on average, 0.6 to 1.14 of the time each:
+// which wave is the last changes with any order; 512 tiles 5.0 -> 3.1, 1024 8.1 -> 4.7).  word[k] is tile k's size and depth; order[p] becomes the
+// tile at place p, offset[p] the sizes of the places before it; returns the sum of all
+// sizes times depths.  Each wave counts, places and adds up a quarter of the tiles.  Every
+// block of the launch does it, so what counts is instructions: 1024 tiles take about 10 us,
+// where counting each tile's place out against all others took 1150 us (256 tiles 76 us).
+struct OrderLds {
+    uint next[4][64];  // per wave and class: tiles, then the next one's place
+    uint64_t sizes[4];
+    float steps[4];
+};
+__device__ float order_by_depth(const uint64_t *word, uint n, OrderLds &lds, ushort *order,
+                                uint64_t *offset) {
+    const uint lane = cu::lane_id(), wave = threadIdx.x >> 6;
+    const uint64_t lanes_below = (1ull << lane) - 1ull;
+    const uint each = (n + 255) / 256 * 64;
+    const uint lo = min(wave * each, n), hi = min(lo + each, n);
+    lds.next[wave][lane] = 0;
+    wave_fence();
+    for (uint k = lo + lane; k < hi; k += 64)
+        atomicAdd(&lds.next[wave][depth_class((uint)(word[k] >> 32))], 1u);
+    __syncthreads();
+    uint count = 0, place = 0;  // of the class `lane`, in all waves and in those before
+#pragma unroll
+    for (uint w = 0; w < 4; ++w) {
+        const uint here = lds.next[w][lane];
+        count += here;
+        if (w < wave) place += here;
+    }
+    uint upto = count;
+#pragma unroll
+    for (uint d = 1; d < 64; d *= 2) {
+        const uint below = __shfl_up(upto, d, 64);
+        if (lane >= d) upto += below;
+    }
+    __syncthreads();
+    lds.next[wave][lane] = upto - count + place;
+    wave_fence();
+    for (uint from = lo; from < hi; from += 64) {
+        const bool have = from + lane < hi;
+        const uint c = have ? depth_class((uint)(word[from + lane] >> 32)) : 0u;
+        uint64_t alike = cu::ballot(have);  // the lanes with a tile of this lane's class
+#pragma unroll
+        for (uint bit = 0; bit < 6; ++bit) {
+            const uint64_t set = cu::ballot((c >> bit) & 1u);
+            alike &= (c >> bit) & 1u ? set : ~set;
+        }
+        const uint at = lds.next[wave][c] + (uint)__popcll(alike & lanes_below);
+        wave_fence();
+        if (have) {
+            order[at] = (ushort)(from + lane);
+            if ((alike >> lane) == 1) lds.next[wave][c] = at + 1;  // its last lane
+        }
+        wave_fence();
+    }
+    __syncthreads();
+    uint64_t base = 0;
+    float steps = 0;
+    for (uint from = lo; from < hi; from += 64) {
+        const bool have = from + lane < hi;
+        const uint64_t w = have ? word[order[from + lane]] : 0u;
+        const uint64_t size = (uint)w;
+        steps += (float)size * (float)(uint)(w >> 32);
+        unsigned long long through = size;
+#pragma unroll
+        for (uint d = 1; d < 64; d *= 2) {
+            const unsigned long long below = __shfl_up(through, d, 64);
+            if (lane >= d) through += below;
+        }
+        if (have) offset[from + lane] = base + through - size;
+        base += __shfl(through, 63, 64);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) steps += __shfl_xor(steps, off, 64);
+    if (lane == 0) {
+        lds.sizes[wave] = base;
+        lds.steps[wave] = steps;
+    }
+    __syncthreads();
+    base = 0;
+    for (uint w = 0; w < wave; ++w) base += lds.sizes[w];
+    for (uint k = lo + lane; k < hi; k += 64) offset[k] += base;
+    return lds.steps[0] + lds.steps[1] + lds.steps[2] + lds.steps[3];
+}
+
 template <class Real, int K, bool kFused>
 __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, uint n_tiles,
                                         uint64_t total, uint *counts, double *smooth,
                                         unsigned long long *iters, unsigned long long *queue,
                                         uint chunk, uint refill) {
     __shared__ uint64_t lds_offset[kMaxLdsTiles];
-    __shared__ double lds_smooth_c[kMaxLdsTiles];
+    __shared__ uint64_t lds_word[kMaxLdsTiles];  // smooth constant; size and depth for order_by_depth
     __shared__ ushort lds_order[kMaxLdsTiles];
-    // The queue runs through the tiles from the deepest max_iter down, so that the longest
-    // orbits do not start last: over 24 batches of tiles of very different depth 3.9 -> 3.2 ms
-    // on average with the smaller grabs below (0.6 to 1.14 of the time each: which wave is
-    // the last changes with any order).  lds_offset holds the places' offsets in that order, and
-    // lds_order their tiles.  Each tile's place is counted out against all others, up to
-    // kMaxSortedTiles of them (a few us); more, and tables that are not a tile after the
-    // other from 0 on, are taken as they come.
-    auto end_of = [&](uint k) { return k + 1 < n_tiles ? tiles[k + 1].work_offset : total; };
-    bool sorted = n_tiles <= kMaxSortedTiles && tiles[0].work_offset == 0;
-    if (sorted) {
-        int broken = 0;
-        for (uint k = threadIdx.x; k < n_tiles; k += blockDim.x)
-            broken |= end_of(k) < tiles[k].work_offset;
-        sorted = __syncthreads_or(broken) == 0;
-    }
-    for (uint k = threadIdx.x; k < n_tiles; k += blockDim.x) {
-        uint64_t offset = tiles[k].work_offset;
-        uint place = k;
-        if (sorted) {
-            const uint depth = tiles[k].max_iter;
-            offset = 0;
-            place = 0;
-            for (uint j = 0; j < n_tiles; ++j) {
-                const uint other = tiles[j].max_iter;
-                if (other > depth || (other == depth && j < k)) {
-                    offset += end_of(j) - tiles[j].work_offset;
-                    ++place;
-                }
-            }
-        }
-        lds_offset[place] = offset;
-        lds_order[place] = (ushort)k;
-        lds_smooth_c[k] = cu::smooth_constant(tiles[k].bailout_sq);
-    }
+    __shared__ OrderLds lds_ordering;
+    __shared__ uint lds_deepest;
+    if (threadIdx.x == 0) lds_deepest = 0;
     __syncthreads();
+    uint deepest = 0;
+    for (uint k = threadIdx.x; k < n_tiles; k += blockDim.x) {
+        const uint64_t offset = tiles[k].work_offset;
+        lds_offset[k] = offset;
+        lds_order[k] = (ushort)k;
+        lds_word[k] = __double_as_longlong(cu::smooth_constant(tiles[k].bailout_sq));
+        deepest = max(deepest, tiles[k].max_iter);
+    }
+    atomicMax(&lds_deepest, deepest);
+    __syncthreads();
+    deepest = __builtin_amdgcn_readfirstlane(lds_deepest);
+    const uint waves = gridDim.x * (blockDim.x >> 6);
+    const uint least = min(chunk, 64u);
+    // The fewest items of a grab at this depth, and a wave's first ones.
+    auto floor_at = [&](uint depth) { return max(min(kGrabSteps / max(depth, 1u), chunk), least); };
+    uint first = floor_at(deepest);
+    if (total < (uint64_t)waves * first && total >> 32 == 0) {
+        const uint spread = deepest < kOrderDepth ? waves : waves / 2u;
+        first = min(first, (((uint)total - 1u) / (spread * 64u) + 1u) * 64u);
+    }
+    const uint64_t first_items = (uint64_t)waves * first;
+    bool in_turn = false;  // the table is a tile after the other from 0 on
+    bool sorted = false;   // and in more than one class
+    float steps = (float)total * (float)deepest;
+    if (first_items < total || deepest >= kOrderDepth) [[unlikely]] {
+        auto size_of = [&](uint k) {
+            return (k + 1 < n_tiles ? tiles[k + 1].work_offset : total) - tiles[k].work_offset;
+        };
+        int broken = lds_offset[0] != 0, uneven = 0;
+        for (uint k = threadIdx.x; k < n_tiles; k += blockDim.x) {
+            broken |= size_of(k) >> 32 != 0;
+            uneven |= depth_class(tiles[k].max_iter) != depth_class(deepest);
+        }
+        in_turn = __syncthreads_or(broken) == 0;
+        sorted = __syncthreads_or(uneven) != 0 && in_turn;
+        if (sorted) {
+            for (uint k = threadIdx.x; k < n_tiles; k += blockDim.x)
+                lds_word[k] = size_of(k) | (uint64_t)tiles[k].max_iter << 32;
+            __syncthreads();
+            steps = order_by_depth(lds_word, n_tiles, lds_ordering, lds_order, lds_offset);
+            __syncthreads();
+            for (uint k = threadIdx.x; k < n_tiles; k += blockDim.x)
+                lds_word[k] = __double_as_longlong(cu::smooth_constant(tiles[k].bailout_sq));
+            __syncthreads();
+        }
+    }
 
     const uint lane = cu::lane_id();
     const uint64_t lanes_below = (1ull << lane) - 1ull;
@@ -246,34 +376,23 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
     // launch does not start with every wave's atomic on the one counter; the counter
     // hands out the items after all of the first ones.  A grab takes `chunk` items
     // while that is at most half of what the launch's waves would each get of the
-    // rest, and fewer towards the end (down to a lane's worth each): one wave's last
-    // 256 pixels of deep orbits would outlast every other wave.  For the same reason the
-    // steps its pixels may take are at most an eighth of a wave's share of the batch's,
-    // and the first items, the deepest, are a lane's worth.
+    // rest, and fewer towards the end: one wave's last 256 pixels of deep orbits would
+    // outlast every other wave.  For the same reason the steps its pixels may take are at
+    // most an eighth of a wave's share of the batch's.  But not fewer than floor_at: the
+    // counter takes an atomic every 12 ns, whatever the number of waves, so grabs of
+    // shallow pixels must not be small.
     const uint64_t wave_global = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) +
                                                                 (threadIdx.x >> 6));
-    const uint waves = gridDim.x * (blockDim.x >> 6);
     const uint share = 33u - __clz(waves);  // log2 of at least twice the waves
-    float steps = 0;                        // an eighth of a wave's share, if sorted
-    if (sorted) {
-        for (uint k = lane; k < n_tiles; k += 64)
-            steps += (float)(end_of(k) - tiles[k].work_offset) * (float)tiles[k].max_iter;
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) steps += __shfl_xor(steps, off, 64);
-        steps /= (float)(8u * waves);
-    }
-    const uint least = min(chunk, 64u);
+    steps /= (float)(8u * waves);             // an eighth of a wave's share
     auto grab_size = [&](uint64_t rest) {
         uint64_t part = rest >> share;
-        if (sorted && rest != 0) {
-            const uint depth = tiles[lds_order[place_of(total - rest)]].max_iter;
-            part = min(part, (uint64_t)cu::first_lane((uint)fminf(steps / (float)max(depth, 1u),
-                                                                  65536.0f)));
-        }
-        return part >= chunk ? chunk : max((uint)part, least);
+        uint depth = deepest;
+        if (sorted && rest != 0) depth = tiles[lds_order[place_of(total - rest)]].max_iter;
+        if (in_turn) part = min(part, (uint64_t)fminf(steps / (float)max(depth, 1u), 65536.0f));
+        const uint size = part >= chunk ? chunk : max((uint)part, floor_at(depth));
+        return (uint)__builtin_amdgcn_readfirstlane(size);
     };
-    const uint first = sorted ? least : grab_size(total);
-    const uint64_t first_items = (uint64_t)waves * first;
     // `left` of the items from `cur` on are this wave's; scalars, so that the branches
     // on them leave the lane masks scalar too.
     uint64_t cur = wave_global * first;
@@ -343,7 +462,8 @@ __device__ void escape_tiles_persistent(const cu_tile_desc *__restrict__ tiles, 
             const cu_tile_desc &t = tiles[tile];
             executed += o.i;
             count_sum += escaped ? o.i : (t.kind == CU_FRACTAL_JULIA ? max_iter : 0u);
-            smooth_sum += escaped ? cu::smooth_value(o.i, (double)mag2, lds_smooth_c[tile]) : 0.0;
+            smooth_sum += escaped ? cu::smooth_value(o.i, (double)mag2,
+                                                      __longlong_as_double(lds_word[tile])) : 0.0;
             ++s;
             if (s < t.spp) {
                 begin_sample<Real>(t, px, py, s, o.x, o.y, o.cx, o.cy);

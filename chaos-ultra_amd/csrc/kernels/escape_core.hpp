@@ -377,7 +377,10 @@ struct LaneOrbit {
 // A block in which no lane changes costs one branch beyond its steps and
 // three compares: while many waves run the loop is bound by VALU issue, but the few
 // waves left with the longest orbits set a launch's length, and a lone wave waits
-// for every scalar instruction.  Whole wave.
+// for every scalar instruction.  It also waits where its 8-byte instructions lie at odd
+// multiples of 4: FP64 batches that end with a few waves' longest orbits took 10 to 18 %
+// longer then.  So the copying form's loop starts at a multiple of 8, from which its
+// steps (all 8 bytes in FP64) are at multiples of 8 too.  Whole wave.
 template <class Real, int K, bool kFused, bool kTurns>
 __device__ __forceinline__ void run_blocks(LaneOrbit<Real> &o, uint64_t &run, uint64_t &failed,
                                            uint64_t &ended, uint64_t counted, uint enough,
@@ -443,6 +446,7 @@ __device__ __forceinline__ void run_blocks(LaneOrbit<Real> &o, uint64_t &run, ui
     } else {
         for (;;) {
             do {
+                asm volatile(".p2align 3");  // see above
                 if (in_mask(run)) {
                     o.sx = o.x;
                     o.sy = o.y;

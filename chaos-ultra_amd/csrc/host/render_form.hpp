@@ -35,17 +35,23 @@ inline bool mostly_inside(const PlaneRect &image, const PlaneRect &old) {
 // One vote group a wave halves what the waves with the most work do and doubles the
 // number of waves, with half of their lanes idle where a pixel takes one sample.  So it
 // is for launches that wait for their longest waves: frames that reuse most of an earlier
-// one (only the fovea and the new edges are sampled), and frames of at most 40 waves a CU
-// in the two-group form.  FP64 at width 1e-4, 4 samples: 1080p zoom frames 420 -> 305 us,
-// 720p 302 -> 208 us; whole frames 640x360 276 -> 189 us, 300x200 221 -> 162 us; the FP32
-// home view 1024x576 209 -> 165 us.  Beyond, frames that fill the GPU with samples lose
-// (a Julia dust 1280x720 at 5 samples 223 -> 230 us, a 4K frame 1521 -> 1818 us), as do
-// single samples (1080p zoom frames 184 -> 207 us).
-inline bool one_group_waves(int64_t width, int64_t height, float max_ss, bool reuse,
-                            const PlaneRect &image, const PlaneRect &old) {
-    if (!(max_ss >= 2.0f)) return false;
-    return (width + 15) / 16 * ((height + 3) / 4) <= 40ll * std::max(1, compute_units()) ||
-           (reuse && mostly_inside(image, old));
+// one (only the fovea and the new edges are sampled), and frames of at most 60 waves a CU
+// in the two-group form.  What it gives there depends on the image, at most half of the
+// longest wave's chain of max_iter steps a sample; what it costs, on its size, however
+// shallow the image (1920x1080 zoom frames 59 -> 81 us, 4K 154 -> 240; a Julia dust of
+// 800x480 143 -> 155).  So max_iter has to be in proportion to the pixels.  Two groups / one,
+// us: FP64 at width 1e-4, maxIter 5000, 4 samples, zoom frames 1080p 368 / 283, 720p 303 /
+// 205, whole frames 720p 318 / 225, 800x480 301 / 194; below the line Julia zoom frames
+// of maxIter 900, 720p 46 / 54, whole ones 800x480 48 / 57, and FP64 4K zooms 550 / 441 the
+// other way.  Over 780 frames (64x48 to 4K, 10 views, 1 to 8 samples) zooms are 5 % faster than
+// with this form always, whole frames even, and none is more than 16 % slower than with two.
+inline bool one_group_waves(int64_t width, int64_t height, float max_ss, uint32_t max_iter,
+                            bool reuse, const PlaneRect &image, const PlaneRect &old) {
+    if (!(max_ss >= 2.0f)) return false;  // single samples: 184 -> 207 us
+    const double pixels = (double)width * (double)height;
+    if (reuse && mostly_inside(image, old)) return pixels <= 800.0 * max_iter;
+    return (width + 15) / 16 * ((height + 3) / 4) <= 60ll * std::max(1, compute_units()) &&
+           pixels <= 400.0 * max_iter;
 }
 
 }  // namespace cu

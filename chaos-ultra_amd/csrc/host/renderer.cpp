@@ -416,7 +416,8 @@ struct RenderKernel {
         const bool reuse = advanced && (flags & CU_FLAG_SAMPLE_REUSE) != 0;
         int rc;
         if (group && strip_rows <= kMaxGridDim &&
-            one_group_waves(width, height, max_ss, reuse, {seg.lbx, seg.lby, seg.rtx, seg.rty},
+            one_group_waves(width, height, max_ss, (uint32_t)max_iterations, reuse,
+                            {seg.lbx, seg.lby, seg.rtx, seg.rty},
                             {origin.lbx, origin.lby, origin.rtx, origin.rty}))
             rc = cu_launch_kernel(group, gx, (unsigned)strip_rows, 1, kBlockDim, kGroupTRows, 1, 0,
                                   params);

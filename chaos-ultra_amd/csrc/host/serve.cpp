@@ -271,7 +271,7 @@ void dispatch(cu_serve_s *s, Session &ss, Slot &sl, const Request &rq) {
             void *params[] = {&out, &pitch, &size, fp32 ? (void *)&rf : (void *)&rd, &maxit,
                               &max_ss, &flags};
             launch_render(fp32 ? s->main_f : s->main_d,
-                          one_group_waves(W, H, max_ss, false, plane, plane), W, H, params, st);
+                          one_group_waves(W, H, max_ss, maxit, false, plane, plane), W, H, params, st);
             path = 1;
         } else {  // renderFast: advanced kernel primary -> secondary, then swap
             void *in = ss.buf[ss.primary];
@@ -288,7 +288,7 @@ void dispatch(cu_serve_s *s, Session &ss, Slot &sl, const Request &rq) {
                               &max_ss, &flags, fp32 ? (void *)&of : (void *)&od, &in, &in_pitch,
                               &focus};
             launch_render(fp32 ? s->adv_f : s->adv_d,
-                          one_group_waves(W, H, max_ss, true, plane,
+                          one_group_waves(W, H, max_ss, maxit, true, plane,
                                           {od.lbx, od.lby, od.rtx, od.rty}),
                           W, H, params, st);
             ss.primary = 1 - ss.primary;

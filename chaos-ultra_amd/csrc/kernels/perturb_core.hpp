@@ -520,9 +520,17 @@ __device__ int perturb_pixel(const OrbitView<Real> &Z, const OrbitInfo &info, Re
     uint m = 0, n_lane = 0;
     int state = active ? 0 : 4;
     mag_out = 0;
+    // Where the reference escapes within a block most pixels do too, and a block with its
+    // replay is the longer way (1080p frames beside the set, FP32 / FP64 55 / 86 -> 26 / 31
+    // us): checked steps until it has.
+    uint n = 0;                          // iterations of the running lanes
+    if (rebase && M < (uint)K)
+        for (; n < M + 2u && cu::ballot(state == 0) != 0; ++n)
+            if (state == 0)
+                state = checked_step<Real>(Z, M, dx, dy, m, n_lane, dcx, dcy, max_iter, bsq, rebase,
+                                           geps, mag_out);
     if (rebase) {
-        uint64_t run = cu::ballot(active), failed = 0;
-        uint n = 0;                      // iterations of the running lanes
+        uint64_t run = cu::ballot(state == 0), failed = 0;
         Real sx = 0, sy = 0;             // block start
         uint sm = 0;
         Real rx = 0, ry = 0;             // delta of the lane's last rebase

@@ -82,3 +82,12 @@ def test_the_bounds_matter(waves):
     *[(CENTRE, 1e-3, k, 6) for k in (1, 31, 32, 33, 63, 64, 65)]])
 def test_frames(waves, precision, centre, width, max_iter, n):
     waves(precision, centre, width, max_iter, n=n)
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("centre,width", [((0.5, 0.5), 0.05), ((-1.2, 0.6), 0.1), ((0.9, 0.9), 0.5), ((0.7, 0.3), 0.01)])
+def test_frames_beside_the_set_take_no_blocks(waves, precision, centre, width):
+    """A reference of a few steps, and pixels that escape with it: one operation a checked
+    step and a few besides, where a block of 32 and its replay take 46."""
+    r = waves(precision, centre, width, 200, n=8)
+    assert r["last"] <= 7 and r["operations"] <= 8 * (r["last"] + 10)

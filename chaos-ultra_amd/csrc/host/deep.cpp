@@ -181,9 +181,9 @@ void launch_pixels(cu_deep d, cu_stream s, DeepArgs &a) {
     // one LDS copy of the reference orbit)
     const uint32_t bw = d->method == CU_DEEP_PERTURB_F64 ? 32 : 16, bh = 16;
     dim3 grid((d->desc.width + bw - 1) / bw, (d->desc.height + bh - 1) / bh, 1);
-    // direct frames of few blocks: 6 per CU (1e-6, maxIter 50000: 9.3 -> 8.9 ms)
-    const bool spread = d->method == CU_DEEP_DIRECT_F64 && few_blocks(grid);
-    launch(d->engine, f, grid, dim3(bw * bh), params, s, false, spread ? lds_for(6) : 0);
+    const bool direct = d->method == CU_DEEP_DIRECT_F64;
+    launch(d->engine, f, grid, dim3(bw * bh), params, s, false,
+           direct ? spread_lds((uint64_t)grid.x * grid.y, 10, 32, 6) : 0);
 }
 
 // The glitched pixel nearest the centroid of all glitched pixels.

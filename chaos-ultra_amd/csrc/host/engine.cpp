@@ -22,11 +22,6 @@ cu_function function(cu_engine e, const std::string &name) {
 
 hipStream_t stream_of(cu_stream s) { return s ? s->stream : nullptr; }
 
-uint32_t lds_for(uint32_t per_cu) {
-    constexpr uint32_t kLdsPerCu = 160u << 10, kGranule = 1280;
-    return kLdsPerCu / per_cu / kGranule * kGranule;
-}
-
 void launch(cu_engine e, cu_function f, dim3 grid, dim3 block, void **params, cu_stream s,
             bool timed, uint32_t lds) {
     hipStream_t st = stream_of(s);
@@ -117,11 +112,6 @@ void fill_u32(cu_engine e, cu_stream s, void *p, uint32_t value, uint64_t words)
     void *params[] = {&p, &value, &words};
     const unsigned blocks = (unsigned)std::min<uint64_t>((words + 255) / 256, 1024);
     launch(e, fn, dim3(blocks), dim3(256), params, s, false);
-}
-
-// At most 32 blocks per CU (lds_for).
-bool few_blocks(dim3 grid) {
-    return (uint64_t)grid.x * grid.y <= 32ull * (uint64_t)std::max(1, compute_units());
 }
 
 bool pick_fused(int variant, const cu_tile_desc &t, int precision) {
@@ -269,12 +259,12 @@ int cu_escape_tile(cu_engine e, int precision, int variant, const cu_tile_desc *
             while ((1u << (lg + 1)) <= ppw) ++lg;
             uint32_t bw = 1u << ((lg + 1) >> 1), bh = ppw / bw;
             dim3 grid((t.width + 2 * bw - 1) / (2 * bw), (t.height + 2 * bh - 1) / (2 * bh), 1);
+            const bool spread = precision == 64 && t.max_iter >= 500;
             launch(e, f, grid, dim3(256, 1, 1), params, stream, true,
-                   few_blocks(grid) ? lds_for(4) : 0);
+                   spread ? spread_lds((uint64_t)grid.x * grid.y, 10, 28, 4) : 0);
         } else {
             dim3 grid((t.width + 15) / 16, (t.height + 15) / 16, 1);
-            launch(e, f, grid, dim3(16, 16, 1), params, stream, true,
-                   few_blocks(grid) ? lds_for(6) : 0);
+            launch(e, f, grid, dim3(16, 16, 1), params, stream, true);
         }
     });
 }

@@ -78,6 +78,7 @@ struct cu_frame_s {
     hipEvent_t ev_start = nullptr, ev_pass1 = nullptr, ev_end = nullptr;
     hipStream_t last_stream = nullptr;
     bool rendered = false;
+    uint32_t deepest = 0;                  // the tiles' largest max_iter
     bool replayed = false;                 // last render was a graph replay (no pass-1 event)
     hipGraph_t graph = nullptr;            // captured render (cu_frame_capture)
     hipGraphExec_t graph_exec = nullptr;
@@ -139,7 +140,6 @@ void enqueue_render(cu_frame f, const cu_frame_tune &tn, const uint32_t *d_palet
     cu_function combine = function(f->engine, "combinePending");
     uint32_t *counters = (uint32_t *)f->d_counters;
     const uint32_t n_tiles = (uint32_t)f->tiles.size();
-    const uint32_t cus = (uint32_t)std::max(1, compute_units());
 
     fill(f, stream, f->d_control, 0, kControlWords);
     if (events) check(hipEventRecord(f->ev_start, st), "hipEventRecord");
@@ -168,10 +168,12 @@ void enqueue_render(cu_frame f, const cu_frame_tune &tn, const uint32_t *d_palet
         uint32_t *c = counters;
         void *params[] = {&a, &total_blocks, &q, &c};
         const uint32_t groups = (total_blocks + 3) / 4;
-        const uint32_t lds = few_blocks(dim3(groups)) ? lds_for(4) : groups <= 64 * cus ? lds_for(5) : 0;
-        launch(f->engine, pass1, dim3(groups), dim3(256), params, stream, false, lds);
+        const bool spread = f->precision == 64 && f->deepest >= 500;
+        launch(f->engine, pass1, dim3(groups), dim3(256), params, stream, false,
+               spread ? spread_lds(groups, 10, 18, 4) : 0);
     }
     if (events) check(hipEventRecord(f->ev_pass1, st), "hipEventRecord");
+    const uint32_t cus = (uint32_t)std::max(1, compute_units());
     // tail passes p = 1..tail_passes: pass p reads queue (p-1) & 1 with fill set
     // p-1 and writes queue p & 1 with fill set p.  Without a drain the last of
     // them runs every orbit to its end; with one, all hand off and the drain
@@ -257,6 +259,7 @@ int cu_frame_create(cu_engine e, const cu_tile_desc *tiles, uint32_t n_tiles, in
             samples += (uint64_t)t.width * t.height * t.spp;
             smooth_c[k] = smooth_constant(t.bailout_sq);
             all_safe = all_safe && fused_safe(t, precision);
+            f->deepest = std::max(f->deepest, t.max_iter);
         }
         uint64_t max_blocks = 0;
         for (uint32_t w = 0; w < kWaveShapes; ++w) {

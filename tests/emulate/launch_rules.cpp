@@ -4,10 +4,15 @@
 //
 // prints the vote groups a wave of the render kernels (1 or 2); `overlap` is the part of the
 // image's width that an earlier one covers.
+//
+//   launch_rules lds <blocks> <from> <to> <per_cu>
+//
+// prints the bytes of LDS that a launch asks for to hold a CU to per_cu blocks.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 
+#include "../../chaos-ultra_amd/csrc/host/engine_helpers.hpp"
 #include "../../chaos-ultra_amd/csrc/host/render_form.hpp"
 
 namespace cu {
@@ -22,6 +27,11 @@ int main(int argc, char **argv) {
                                                 atoi(argv[6]) != 0, image, old)
                                 ? 1
                                 : 2);
+        return 0;
+    }
+    if (argc == 6 && std::strcmp(argv[1], "lds") == 0) {
+        std::printf("%u\n", cu::spread_lds(strtoull(argv[2], nullptr, 10), (uint32_t)atoi(argv[3]),
+                                           (uint32_t)atoi(argv[4]), (uint32_t)atoi(argv[5])));
         return 0;
     }
     return 2;

@@ -37,3 +37,12 @@ def rule(tmp_path_factory):
     ((800, 480), 1, 5000, 0, 0, 2)])
 def test_render_forms(rule, size, samples, max_iter, reuse, overlap, groups):
     assert rule("forms", *size, samples, max_iter, reuse, overlap) == groups
+
+
+@pytest.mark.parametrize("blocks,per_cu,bytes_", [
+    (1, 4, 0), (4 * 256, 4, 0), (10 * 256 - 1, 4, 0), (10 * 256, 4, 40960), (28 * 256, 4, 40960),
+    (28 * 256 + 1, 4, 0), (10 * 256, 6, 26880), (1 << 40, 4, 0)])
+def test_unused_lds(rule, blocks, per_cu, bytes_):
+    """Asked for only by launches of 10 to 28 blocks per CU: it keeps other streams' kernels off
+    the CUs, and smaller launches have nothing to hold back."""
+    assert rule("lds", blocks, 10, 28, per_cu) == bytes_

@@ -379,8 +379,9 @@ struct LaneOrbit {
 // waves left with the longest orbits set a launch's length, and a lone wave waits
 // for every scalar instruction.  It also waits where its 8-byte instructions lie at odd
 // multiples of 4: FP64 batches that end with a few waves' longest orbits took 10 to 18 %
-// longer then.  So the copying form's loop starts at a multiple of 8, from which its
-// steps (all 8 bytes in FP64) are at multiples of 8 too.  Whole wave.
+// longer then, a 100x60 tile of maxIter 3000 6 % (80.7 us, 76.1 aligned; frames that fill the
+// GPU are even).  So a block starts at a multiple of 8, from which its steps (all 8 bytes in
+// FP64) are at multiples of 8 too.  Whole wave.
 template <class Real, int K, bool kFused, bool kTurns>
 __device__ __forceinline__ void run_blocks(LaneOrbit<Real> &o, uint64_t &run, uint64_t &failed,
                                            uint64_t &ended, uint64_t counted, uint enough,
@@ -391,6 +392,7 @@ __device__ __forceinline__ void run_blocks(LaneOrbit<Real> &o, uint64_t &run, ui
     uint64_t turned = 0;  // lanes that ended with their state in (sx, sy)
     uint64_t inside, due, again;
     auto block = [&](const Real &fx, const Real &fy, Real &tx, Real &ty) {
+        asm volatile(".p2align 3");  // see above
         if (in_mask(run)) {
             Real x = fx, y = fy;
 #pragma unroll

@@ -31,25 +31,11 @@ namespace cu {
 __device__ __forceinline__ float fma_r(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_r(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// One step.  kFused computes y' as fma(x*y, 2, cy): 2*(x*y) is exact, so this
-// equals ((2x)*y)+cy whenever x*y is zero or at least the smallest normal —
-// one VALU op fewer (6 per step instead of 7).
-template <class Real, bool kFused>
-__device__ __forceinline__ void quad_step(Real &x, Real &y, Real cx, Real cy) {
-    const Real x2 = x * x;
-    const Real y2 = y * y;
-    const Real xn = (x2 - y2) + cx;
-    if constexpr (kFused) {
-        y = fma_r(x * y, (Real)2, cy);
-    } else {
-        y = ((x + x) * y) + cy;
-    }
-    x = xn;
-}
-
-// One step with the squares carried: (x2, y2) hold x*x and y*y of the current
-// state on entry and of the new state on exit, so a block-end test reads them
-// instead of recomputing them.  Same operations and roundings as quad_step.
+// One step, with the squares carried: (x2, y2) hold x*x and y*y of the current state on
+// entry and of the new state on exit, so a block-end test reads them instead of
+// recomputing them.  kFused computes y' as fma(x*y, 2, cy): 2*(x*y) is exact, so this
+// equals ((2x)*y)+cy whenever x*y is zero or at least the smallest normal — one VALU op
+// fewer (6 per step instead of 7).
 template <class Real, bool kFused>
 __device__ __forceinline__ void quad_step_sq(Real &x, Real &y, Real &x2, Real &y2, Real cx,
                                              Real cy) {

@@ -100,7 +100,7 @@ __device__ void escape_tile(const cu_tile_desc &t, double smooth_c, uint *counts
 // Bound by the waves with the longest orbits and how they share out over the SIMDs
 // (VALU issue 0.39).  Whole set, 1024^2, maxIter 1000, FP64, kernel alone 92 -> 71 us
 // with the cycle test (0.41 of the loop's steps left, 0.6 of its longest orbits per
-// wave) and 62 us with run_blocks' loop and 4 blocks per CU (lds_for); 777x613 FP32
+// wave) and 62 us with run_blocks' loop and 4 blocks per CU (spread_lds); 777x613 FP32
 // Julia set, 3 spp (escape_tile) with compose 74-95 -> 39-50 us.  Tried and not kept: a
 // wave taking 2 to 4 blocks as one pool whose lanes refill (101 us: a wave then runs
 // several long orbits one after another).

@@ -21,14 +21,15 @@ extern "C" __global__ __launch_bounds__(64) void referenceOrbitDouble(
 // it can go through the scalar cache.  The second bound (8 waves per SIMD)
 // keeps the kernels within 64 VGPRs, so that a CU's 32 wave slots can all be
 // filled; without it the compiler keeps a whole block's orbit reads in flight.
-// Blocks of 32 steps.  Block shapes: perturb_frame.
+// Steps a block: kPlainSteps, the length that the orbit's bounds are for.  Block shapes:
+// perturb_frame.
 extern "C" __global__ __launch_bounds__(256, 8) void perturbFloat(
     DeepArgs a, const OrbitEntry<float> *__restrict__ orbit) {
-    perturb_frame<float, 32, 2, 2, 20u * 1024u>(a, orbit);
+    perturb_frame<float, kPlainSteps, 2, 2, 20u * 1024u>(a, orbit);
 }
 extern "C" __global__ __launch_bounds__(512, 8) void perturbDouble(
     DeepArgs a, const OrbitEntry<double> *__restrict__ orbit) {
-    perturb_frame<double, 32, 4, 2, 40u * 1024u>(a, orbit);
+    perturb_frame<double, kPlainSteps, 4, 2, 40u * 1024u>(a, orbit);
 }
 extern "C" __global__ __launch_bounds__(256) void deepDirectDoubleExact(DeepArgs a) {
     deep_direct<16, false>(a);

@@ -621,10 +621,10 @@ CU_RENDER_KERNELS(, __launch_bounds__(1024), __launch_bounds__(1024), 16u, 2u)
 // The same kernels for 32 x 4-thread blocks over ceil(W/32) x ceil(H/4), which
 // the renderer layer and the serving loop launch: the same pixels, vote groups
 // and results.  A 1024-thread block's LDS and wave slots free only when its last
-// wave ends, and with 70 VGPRs a CU holds 28 waves, so the next such block waits
+// wave ends, and with 72 VGPRs a CU holds 28 waves, so the next such block waits
 // for 4 of them: about 3 waves per SIMD stay resident.  Blocks of 2 waves keep
 // the wave slots filled (14 blocks per CU, 136 KB of LDS).  The FP64 advanced
-// kernel needs 78 VGPRs: it is held to 6 waves per SIMD rather than spill.
+// kernel needs 80 VGPRs: it is held to 6 waves per SIMD rather than spill.
 CU_RENDER_KERNELS(Strip, __launch_bounds__(128, 7), __launch_bounds__(128, 6), 2u, 2u)
 
 // One vote group a wave, 32 x 8-thread blocks over the same grid as *Strip, for launches

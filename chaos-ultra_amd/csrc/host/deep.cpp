@@ -9,6 +9,7 @@
 
 #include "common.hpp"
 #include "engine_helpers.hpp"
+#include "glitch_pick.hpp"
 #include "handles.hpp"
 
 namespace {
@@ -186,34 +187,6 @@ void launch_pixels(cu_deep d, cu_stream s, DeepArgs &a) {
            direct ? spread_lds((uint64_t)grid.x * grid.y, 10, 32, 6) : 0);
 }
 
-// The glitched pixel nearest the centroid of all glitched pixels.
-bool pick_secondary(const std::vector<unsigned char> &flags, uint32_t W, uint32_t H, uint32_t &px,
-                    uint32_t &py, uint32_t &count) {
-    double sx = 0, sy = 0;
-    count = 0;
-    for (uint32_t y = 0; y < H; ++y)
-        for (uint32_t x = 0; x < W; ++x)
-            if (flags[(size_t)y * W + x]) {
-                sx += x;
-                sy += y;
-                ++count;
-            }
-    if (count == 0) return false;
-    const double cx = sx / count, cy = sy / count;
-    double best = -1;
-    for (uint32_t y = 0; y < H; ++y)
-        for (uint32_t x = 0; x < W; ++x)
-            if (flags[(size_t)y * W + x]) {
-                const double d2 = (x - cx) * (x - cx) + (y - cy) * (y - cy);
-                if (best < 0 || d2 < best) {
-                    best = d2;
-                    px = x;
-                    py = y;
-                }
-            }
-    return true;
-}
-
 }  // namespace
 }  // namespace cu
 
@@ -336,7 +309,7 @@ int cu_deep_render(cu_deep d, const uint32_t *d_palette, uint32_t palette_length
                 check(hipMemcpy(flags.data(), d->d_glitch, pixels, hipMemcpyDeviceToHost),
                       "hipMemcpy D2H");
                 uint32_t px = 0, py = 0, count = 0;
-                if (!pick_secondary(flags, c.width, c.height, px, py, count)) break;
+                if (!pick_secondary(flags.data(), c.width, c.height, px, py, count)) break;
                 d->glitched = count;
                 if (r >= c.max_references) break;
                 const double ox = ((double)px + 0.5 - (double)c.width * 0.5) * c.pixel_w;
